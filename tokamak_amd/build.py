@@ -21,7 +21,7 @@ LIB_PATH = os.path.join(PKG, LIB_NAME)
 # The runtime library: everything of libtkm_attn.so plus the tkm.h runtime (tkm_hip.c), the
 # whole-graph generator, the hipBLASLt GEMMs and the runtime's kernels.
 HIP_LIB_PATH = os.path.join(PKG, "libtkm_hip.so")
-RT_SOURCES = ["tkm_gemm.hip", "tkm_rt_kernels.hip"]
+RT_SOURCES = ["tkm_gemm.hip", "tkm_gemm_mfma.hip", "tkm_rt_kernels.hip"]
 RT_C_SOURCES = ["tkm_codegen_hip.c", "tkm_hip.c"]
 SOURCES = ["attn_fwd.hip", "attn_asm.hip", "attn_bwd.hip", "tkm_attn_abi.hip"]
 # Hand-scheduled assembly kernels: (generator module, kernel symbol).  Each is generated,

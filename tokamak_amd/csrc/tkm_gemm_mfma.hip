@@ -1,0 +1,396 @@
+// tkm_gemm_mfma.hip -- the runtime's FC GEMMs on gfx950 matrix cores.
+//
+//   C[m][n] = sum_k A(m, k) B(k, n)  (+ C[m][n]),  fp32 accumulation, row-major C
+//
+// for the three products of an FC layer, none of which needs a transposed copy:
+//   forward  out[rows][N] = in[rows][K] W[K][N]        A along k (KC), B along n (NC)
+//   dX       din[rows][K] = dout[rows][N] W[K][N]^T    A along k,      B along k
+//   dW       dW[K][N]     = in[rows][K]^T dout[rows][N] A along m (NC), B along n
+// An operand stored along k ("KC", [index][k]) is read from LDS 16 bytes per lane, the MFMA's own
+// layout; one stored along its output index ("NC", [k][index]) is read with the transposing
+// ds_read_b64_tr_b16.  Tiles go HBM -> LDS by DMA and are swizzled as the attention kernels'
+// (attn_common.h), which keeps both kinds of reads free of bank conflicts.
+//
+// What bounds them: with 4096 rows and K, N of 512 to 2752 a 128x128 tile runs 8 to 43 steps of 64 k, so
+// the latency of the first loads and the fill of the chip by few tiles weigh as much as the matrix rate;
+// and the transposing reads deliver half the bytes per cycle, so dW (both operands NC) is bound by LDS
+// reads.  Hence several tile sizes (pick_tile), STAGES k-steps of LDS with STAGES - 1 in flight, a fixed
+// place for every LDS read and request between the MFMAs (in one burst they hold the wave's issue: dW
+// K 4096, N 8192: 65 -> 46 us), and the DMA issued from inline assembly (behind the DMA builtin the compiler
+// waits for every load in flight before each batch of transposed reads).
+// Measured in bf16 at rows 4096, against hipBLASLt's first choice in the same training step:
+//   forward  N 1536, K 512 : 12.8 us (17.5)     dX  N 512, K 1536 : 12.1 us (24.5)
+//            N 512,  K 512 :  7.2 us (12.8)         N 512, K 512  :  6.9 us (10.4)
+//            N 2752, K 512 : 20.0 us (30)           N 512, K 2752 : 19.4 us (44)
+//            N 512, K 1376 : 12.0 us (21.3)         N 1376, K 512 : 11.4 us (31)
+//            N 8192, K 512 : 57 us (50)             N 512, K 8192 : 53 us (118)
+// and 4096 x 4096 x 4096 at 1.04 PFLOP/s (256x128).  The 8-layer decoder's training step: 3676 -> 2910 us,
+// outputs equal bit for bit (the MFMA sums run over k in the same order).
+//
+// A workgroup is 4 waves in a 2 x 2 grid.  The product is formed transposed (the B operand's columns
+// are the MFMA's rows), so a lane holds one row of C and 4 consecutive columns per register quad;
+// the tile leaves through LDS as fp32 rows, read back as whole 16-byte groups of columns.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "attn_common.h"
+#include "tkm_gemm_mfma.h"
+
+namespace {
+
+using namespace tkm;
+
+constexpr int BK = 64, KST = BK / 16;   // k of one step, its MFMA k-groups
+
+// Buffer descriptor as four scalar words (for inline assembly).
+__device__ __forceinline__ u32x4 desc(const char* base, long long bytes) {
+    const uint64_t p = (uint64_t)base;
+    const uint32_t n = bytes <= 0 ? 0u : (bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes);
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((p >> 32) & 0xffffu)),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
+}
+
+// 16 bytes per lane from descriptor + voff to LDS at lds + 16 * lane.  No register is written; the
+// compiler does not see the load, so each step waits for it explicitly (wait_step).
+// FIRST: the descriptor may have just been written by a VALU lane read, which a buffer access may
+// follow only after 5 wait states; otherwise one, between the write of m0 and its use.
+template <bool FIRST>
+__device__ __forceinline__ void dma_asm(u32x4 d, uint32_t lds, uint32_t voff) {
+    if constexpr (FIRST)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(lds), "v"(voff), "s"(d));
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(lds), "v"(voff), "s"(d));
+}
+
+// Until at most N of this wave's DMA requests are in flight and its LDS reads are done, then the
+// workgroup's barrier: after it every wave's share of the awaited tile is in LDS.
+template <int N>
+__device__ __forceinline__ void wait_step() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+}
+
+// LDS layout of one operand tile.  KC: IDX rows of BK values; NC: BK rows of IDX values (IDX <= 128).
+template <bool KC, int IDX>
+struct Operand {
+    static constexpr int ROWS = KC ? IDX : BK, COLS = KC ? BK : IDX;
+    static constexpr int ROWB = COLS * 2, CPR = COLS / 8, BYTES = ROWS * ROWB;
+    static constexpr int RPI = 64 / CPR, NI = ROWS / RPI / 4;   // rows per DMA request, requests per wave
+    static_assert(COLS == 64 || COLS == 128 || COLS == 256, "tile rows of 128 or 256 bytes");
+    static __device__ __forceinline__ int swizzle(int r) { return swz<(COLS > 128 ? 128 : COLS)>(r); }
+};
+
+template <int DT, bool AKC, bool BKC, int BM, int BN, int STAGES, bool OUT32>
+struct Gemm {
+    using TA = Operand<AKC, BM>;
+    using TB = Operand<BKC, BN>;
+    static constexpr int WM = BM / 2, WN = BN / 2, MB = WM / 32, NB = WN / 32;
+    static constexpr int NDMA = TA::NI + TB::NI;
+    static constexpr int STAGE_BYTES = TA::BYTES + TB::BYTES;
+    static constexpr int EPITCH = WN + 4;                       // fp32 staging row
+    static constexpr int EPI_BYTES = 4 * 32 * EPITCH * 4;
+    static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > EPI_BYTES ? STAGES * STAGE_BYTES : EPI_BYTES;
+
+    // LDS reads of one MFMA operand (32 indices from idx0, 16 k of step ks): one of 16 bytes per lane
+    // (KC) or two transposing ones of 8 (NC).
+    template <bool KC>
+    static constexpr int PIECES = KC ? 1 : 2;
+    template <class T, bool KC>
+    static __device__ __forceinline__ void piece(u32x4& x, const char* t, int idx0, int ks, int tt, int lane) {
+        const int l32 = lane & 31, hi = lane >> 5;
+        if constexpr (KC) {
+            const int r = idx0 + l32;
+            x = ld_lds16((const uint16_t*)(t + r * T::ROWB + (((ks * 2 + hi) ^ T::swizzle(l32)) << 4)));
+        } else {
+            const int row = ks * 16 + hi * 8 + tt * 4 + ((lane & 15) >> 2);
+            const int col = idx0 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+            const u32x2 v = ld_lds_tr(t + row * T::ROWB + (((col >> 3) ^ T::swizzle(row)) << 4) + (col & 7) * 2);
+            x[2 * tt] = v[0];
+            x[2 * tt + 1] = v[1];
+        }
+    }
+
+    static __device__ __forceinline__ void run(const TkmGemmProblem& p, int tm, int tn, int accumulate, char* smem) {
+        const int tid = threadIdx.x, lane = tid & 63;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int m0 = tm * BM, n0 = tn * BN;
+        const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
+        const int nt = (p.K + BK - 1) / BK;
+
+        // Bytes from one k-step's tile to the next, and from the tile's first byte to the tensor's end.
+        const long long pa = 2ll * p.lda, pb = 2ll * p.ldb;
+        const char* abase = (const char*)p.A + (AKC ? (long long)m0 * pa : 2ll * m0);
+        const char* bbase = (const char*)p.B + (BKC ? (long long)n0 * pb : 2ll * n0);
+        const long long aend = AKC ? (p.M - 1ll - m0) * pa + 2ll * p.K : (p.K - 1ll) * pa + 2ll * (p.M - m0);
+        const long long bend = BKC ? (p.N - 1ll - n0) * pb + 2ll * p.K : (p.K - 1ll) * pb + 2ll * (p.N - n0);
+        const long long astep = AKC ? 2ll * BK : BK * pa, bstep = BKC ? 2ll * BK : BK * pb;
+
+        // This lane's global offset for each of its wave's requests, and its chunk's first k (KC).
+        uint32_t va[TA::NI], vb[TB::NI];
+        const int ra = lane / TA::CPR, ca = lane % TA::CPR, rb = lane / TB::CPR, cb = lane % TB::CPR;
+#pragma unroll
+        for (int i = 0; i < TA::NI; ++i) {
+            const int r = (wave * TA::NI + i) * TA::RPI + ra;
+            va[i] = (uint32_t)r * (uint32_t)pa + (uint32_t)((ca ^ TA::swizzle(r)) << 4);
+        }
+#pragma unroll
+        for (int i = 0; i < TB::NI; ++i) {
+            const int r = (wave * TB::NI + i) * TB::RPI + rb;
+            vb[i] = (uint32_t)r * (uint32_t)pb + (uint32_t)((cb ^ TB::swizzle(r)) << 4);
+        }
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+
+        // The requests of one step's tile, one at a time (q = 0 .. NDMA - 1).
+        struct Tile {
+            u32x4 da, db;
+            uint32_t lds;
+            int left;       // k left from this step on (chunks past K come from out of range, as zeros)
+        };
+        auto tile_at = [&](int t, int buf) __attribute__((always_inline)) {
+            return Tile{desc(abase + t * astep, aend - t * astep), desc(bbase + t * bstep, bend - t * bstep),
+                        lds0 + buf * STAGE_BYTES, p.K - t * BK};
+        };
+        auto request = [&](const Tile& x, int q) __attribute__((always_inline)) {
+            if (q < TA::NI) {
+                uint32_t v = va[q];
+                if constexpr (AKC) {
+                    const int r = (wave * TA::NI + q) * TA::RPI + ra;
+                    if (x.left < BK) v = ((ca ^ TA::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
+                }
+                if (q == 0) dma_asm<true>(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
+                else dma_asm<false>(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
+            } else {
+                const int i = q - TA::NI;
+                uint32_t v = vb[i];
+                if constexpr (BKC) {
+                    const int r = (wave * TB::NI + i) * TB::RPI + rb;
+                    if (x.left < BK) v = ((cb ^ TB::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
+                }
+                if (i == 0) dma_asm<true>(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
+                else dma_asm<false>(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
+            }
+        };
+
+        f32x16 acc[MB][NB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc[i][j] = f32x16{};
+
+        // Operands of one k-step in registers.  Those of (step t + 1, k-group g) are read from LDS once the
+        // MFMAs of (t, g) have gone out, 2 to 3 k-groups ahead of their use, into the same registers.  A
+        // wave issues in order and stalls while the LDS or request queues are full, so the reads and the
+        // DMA requests are dealt out between the MFMAs, slot by slot.
+        u32x4 xa[KST][MB], xb[KST][NB];
+        constexpr int PA = PIECES<AKC>, PB = PIECES<BKC>, NRK = MB * PA + NB * PB;   // reads per k-group
+        constexpr int KSLOT = MB * NB, NSLOT = KST * KSLOT;                          // MFMAs per k-group, per step
+        constexpr int MEET = KSLOT + (KSLOT + 1) / 2, REST = NSLOT - MEET;           // slot of the barrier, slots after
+        auto read = [&](int stage, int ks, int q) __attribute__((always_inline)) {
+            const char* at = smem + stage * STAGE_BYTES;
+            if (q < MB * PA) piece<TA, AKC>(xa[ks][q / PA], at, wm + (q / PA) * 32, ks, q % PA, lane);
+            else {
+                const int u = q - MB * PA;
+                piece<TB, BKC>(xb[ks][u / PB], at + TA::BYTES, wn + (u / PB) * 32, ks, u % PB, lane);
+            }
+        };
+
+#pragma unroll
+        for (int t = 0; t < STAGES; ++t) {
+            const Tile tl = tile_at(t, t);
+#pragma unroll
+            for (int q = 0; q < NDMA; ++q) request(tl, q);
+        }
+        wait_step<(STAGES - 1) * NDMA>();
+#pragma unroll
+        for (int r = 0; r < (KST - 1) * NRK; ++r) read(0, r / NRK, r % NRK);
+        // Past the last step the requests are out of range (zeros into a stage nobody reads) and the
+        // reads unused: every step has the same instructions and the same number in flight.
+        int buf = 0;
+        for (int t = 0; t < nt; ++t) {
+            const int next = buf + 1 == STAGES ? 0 : buf + 1;
+            const Tile tl = tile_at(t + STAGES, buf);
+#pragma unroll
+            for (int s = 0; s < NSLOT; ++s) {
+                const int ks = s / KSLOT, i = (s / NB) % MB, j = s % NB;
+                // every wave has read stage t, and tile t + 1 is in LDS
+                if (s == MEET) wait_step<(STAGES - 2) * NDMA>();
+                acc[i][j] = mfma32<DT>(xb[ks][j], xa[ks][i], acc[i][j]);
+                if (s < KSLOT) {
+#pragma unroll
+                    for (int r = s * NRK / KSLOT; r < (s + 1) * NRK / KSLOT; ++r) read(buf, KST - 1, r);
+                }
+                if (s >= MEET) {
+                    const int u = s - MEET;
+                    constexpr int NR = (KST - 1) * NRK;
+#pragma unroll
+                    for (int r = u * NR / REST; r < (u + 1) * NR / REST; ++r) read(next, r / NRK, r % NRK);
+#pragma unroll
+                    for (int q = u * NDMA / REST; q < (u + 1) * NDMA / REST; ++q) request(tl, q);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            buf = next;
+        }
+        wait_step<0>();
+
+        // acc[i][j]: lane row wm + i*32 + l32, columns wn + j*32 + g4*8 + hi*4 + 0..3 of register quad g4.
+        const int l32 = lane & 31, hi = lane >> 5;
+        float* st = reinterpret_cast<float*>(smem) + wave * 32 * EPITCH;
+        constexpr int VEC = OUT32 ? 4 : 8, CPW = WN / VEC, RPP = 64 / CPW;   // columns a lane stores, lanes per row
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int g4 = 0; g4 < 4; ++g4)
+                    *reinterpret_cast<f32x4*>(st + l32 * EPITCH + j * 32 + g4 * 8 + hi * 4) =
+                        f32x4{acc[i][j][g4 * 4], acc[i][j][g4 * 4 + 1], acc[i][j][g4 * 4 + 2], acc[i][j][g4 * 4 + 3]};
+            // one wave's LDS operations complete in order: its own rows need no wait beyond the reads'
+#pragma unroll
+            for (int q = 0; q < 32 / RPP; ++q) {
+                const int r = q * RPP + lane / CPW, c = (lane % CPW) * VEC;
+                const int m = m0 + wm + i * 32 + r, n = n0 + wn + c;
+                const f32x4 x = *reinterpret_cast<const f32x4*>(st + r * EPITCH + c);
+                if constexpr (OUT32) {
+                    if (m < p.M && n < p.N) *reinterpret_cast<f32x4*>((float*)p.C + (size_t)m * p.ldc + n) = x;
+                } else {
+                    const f32x4 y = *reinterpret_cast<const f32x4*>(st + r * EPITCH + c + 4);
+                    if (m < p.M && n < p.N) {
+                        uint16_t* cp = (uint16_t*)p.C + (size_t)m * p.ldc + n;
+                        float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+                        if (accumulate) {
+                            const u32x4 old = ld_global16(cp);
+#pragma unroll
+                            for (int w = 0; w < 4; ++w) {
+                                const uint32_t o = old[w];
+                                v[2 * w] += to_f32<DT>((uint16_t)(o & 0xffffu));
+                                v[2 * w + 1] += to_f32<DT>((uint16_t)(o >> 16));
+                            }
+                        }
+                        *reinterpret_cast<u32x4*>(cp) = u32x4{pack2<DT>(v[0], v[1]), pack2<DT>(v[2], v[3]),
+                                                              pack2<DT>(v[4], v[5]), pack2<DT>(v[6], v[7])};
+                    }
+                }
+            }
+        }
+    }
+};
+
+// Workgroup w runs on XCD w % 8: each XCD takes a contiguous run of tiles, so the tiles that share an
+// operand's rows share one L2.
+__device__ __forceinline__ int xcd_tile(int w, int n) {
+    const int x = w & 7, q = n >> 3, r = n & 7;
+    return x * q + (x < r ? x : r) + (w >> 3);
+}
+
+template <int DT, bool AKC, bool BKC, int BM, int BN, int STAGES, bool OUT32>
+__global__ __launch_bounds__(256, BM * BN * STAGES >= 65536 ? 1 : 2)
+void k_gemm(TkmGemmProblem p, int accumulate) {
+    using G = Gemm<DT, AKC, BKC, BM, BN, STAGES, OUT32>;
+    __shared__ __attribute__((aligned(1024))) char smem[G::LDS_BYTES];
+    const int tiles_n = (p.N + BN - 1) / BN;
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    G::run(p, t / tiles_n, t % tiles_n, accumulate, smem);
+}
+
+// Several weight gradients in one launch: the table gives each problem's first tile.
+template <int DT, int BM, int BN, int STAGES>
+__global__ __launch_bounds__(256, BM * BN * STAGES >= 65536 ? 1 : 2)
+void k_gemm_group(const TkmGemmProblem* __restrict__ table, int np) {
+    using G = Gemm<DT, false, false, BM, BN, STAGES, true>;
+    __shared__ __attribute__((aligned(1024))) char smem[G::LDS_BYTES];
+    const int w = xcd_tile(blockIdx.x, gridDim.x);
+    int lo = 0, hi = np - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (table[mid].tile0 <= w) lo = mid; else hi = mid - 1;
+    }
+    const TkmGemmProblem p = table[lo];
+    const int t = w - p.tile0, tiles_n = (p.N + BN - 1) / BN;
+    G::run(p, t / tiles_n, t % tiles_n, 0, smem);
+}
+
+long long tiles_of(const TkmGemmProblem& p, int bm, int bn) {
+    return (long long)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn);
+}
+
+int status() { return hipGetLastError() == hipSuccess ? 0 : -1; }
+
+template <int DT, bool BKC, int BM, int BN, int STAGES>
+int launch_t(const TkmGemmProblem& p, int accumulate, hipStream_t s) {
+    hipLaunchKernelGGL((k_gemm<DT, true, BKC, BM, BN, STAGES, false>), dim3((unsigned)tiles_of(p, BM, BN)), dim3(256), 0,
+                       s, p, accumulate);
+    return status();
+}
+
+// Tile of one product, measured at rows 4096 in bf16 (us at 256x128, 128x128, 128x64, 64x64):
+//   N 8192, K 512 : 55, 66, 68, 97      four tiles of 256x128 a CU: the LDS reads of a larger wave
+//   N 2752, K 512 : 23, 20, 25, 35      tile (128x64) are the cheapest
+//   N 1536, K 512 : 13, 13, 15, 20      fewer tiles than that leave CUs idle in the last round
+//   N 512, K 2752 : 34, 30, 19, 25      128 tiles of 128x128 leave half the chip idle
+//   N 512, K 512  : 11, 8.4, 7.3, 7.6
+// and rows 200, N 512, K 2752 (where a step's latency counts): 32, 22, 18, 15.
+int pick_tile(const TkmGemmProblem& p) {
+    if (tiles_of(p, 256, 128) >= 512) return TKM_GEMM_TILE_256x128;
+    if (tiles_of(p, 128, 128) >= 320) return TKM_GEMM_TILE_128x128;
+    return tiles_of(p, 128, 64) >= 192 ? TKM_GEMM_TILE_128x64 : TKM_GEMM_TILE_64x64;
+}
+
+template <int DT, bool BKC>
+int launch_tile(const TkmGemmProblem& p, int tile, int accumulate, hipStream_t s) {
+    switch (tile < 0 ? pick_tile(p) : tile) {
+        case TKM_GEMM_TILE_256x128: return launch_t<DT, BKC, 256, 128, 3>(p, accumulate, s);
+        case TKM_GEMM_TILE_128x128: return launch_t<DT, BKC, 128, 128, 2>(p, accumulate, s);
+        case TKM_GEMM_TILE_128x64: return launch_t<DT, BKC, 128, 64, 3>(p, accumulate, s);
+        default: return launch_t<DT, BKC, 64, 64, 4>(p, accumulate, s);
+    }
+}
+
+template <int DT>
+int launch_group(const TkmGemmProblem* d, int n, long long tiles, int tile, hipStream_t s) {
+    if (tile == TKM_GEMM_TILE_256x128)
+        hipLaunchKernelGGL((k_gemm_group<DT, 256, 128, 3>), dim3((unsigned)tiles), dim3(256), 0, s, d, n);
+    else if (tile == TKM_GEMM_TILE_128x128)
+        hipLaunchKernelGGL((k_gemm_group<DT, 128, 128, 4>), dim3((unsigned)tiles), dim3(256), 0, s, d, n);
+    else
+        hipLaunchKernelGGL((k_gemm_group<DT, 64, 64, 4>), dim3((unsigned)tiles), dim3(256), 0, s, d, n);
+    return status();
+}
+
+}  // namespace
+
+extern "C" {
+
+int tkm_gemm_mfma_supported(const TkmGemmProblem* p, int weight_grad) {
+    if (p->M < 1 || p->N < 1 || p->K < 1 || p->N % 8 || p->lda % 8 || p->ldb % 8 || p->ldc % 8) return 0;
+    if (weight_grad ? p->M % 8 : p->K % 8) return 0;
+    const long long lim = 1ll << 30;    // offsets of 256 stored rows, formed in 32 bits
+    return 512ll * p->lda < lim && 512ll * p->ldb < lim && tiles_of(*p, 64, 64) < (1ll << 31);
+}
+
+int tkm_gemm_mfma_run(const TkmGemmProblem* p, int b_along_k, int bf16, int tile, int accumulate, void* stream) {
+    hipStream_t s = (hipStream_t)stream;
+    if (bf16)
+        return b_along_k ? launch_tile<DT_BF16, true>(*p, tile, accumulate, s)
+                         : launch_tile<DT_BF16, false>(*p, tile, accumulate, s);
+    return b_along_k ? launch_tile<DT_F16, true>(*p, tile, accumulate, s)
+                     : launch_tile<DT_F16, false>(*p, tile, accumulate, s);
+}
+
+long long tkm_gemm_mfma_tiles(const TkmGemmProblem* p, int tile) {
+    return tile == TKM_GEMM_TILE_256x128   ? tiles_of(*p, 256, 128)
+           : tile == TKM_GEMM_TILE_128x128 ? tiles_of(*p, 128, 128)
+                                           : tiles_of(*p, 64, 64);
+}
+
+int tkm_gemm_mfma_group(const TkmGemmProblem* table, int n, long long tiles, int bf16, int tile, void* stream) {
+    if (n <= 0 || tiles <= 0) return 0;
+    return bf16 ? launch_group<DT_BF16>(table, n, tiles, tile, (hipStream_t)stream)
+                : launch_group<DT_F16>(table, n, tiles, tile, (hipStream_t)stream);
+}
+
+}  // extern "C"

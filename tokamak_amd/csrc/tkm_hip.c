@@ -8,10 +8,10 @@
  *   load / step / eval / forward / probes / I/O      tkm_gpu.cu:1423-1999
  *
  * with this build's kernels: the generated qkv-prep and plasma epilogues (tkm_codegen_hip.c,
- * compiled by hipRTC for gfx950), the attention kernels (include/tkm_attn.h), hipBLASLt GEMMs
- * (tkm_gemm.hip) and the runtime's own kernels (tkm_rt_kernels.hip).  The step is captured
- * once into a hipGraph and replayed, as the reference does.  Host code is C; HIP is called
- * through its C API.
+ * compiled by hipRTC for gfx950), the attention kernels (include/tkm_attn.h), the FC GEMMs
+ * (tkm_gemm_mfma.hip, or hipBLASLt through tkm_gemm.hip for the shapes it does not take) and the
+ * runtime's own kernels (tkm_rt_kernels.hip).  The step is captured once into a hipGraph and
+ * replayed, as the reference does.  Host code is C; HIP is called through its C API.
  *
  * Scope: the transformer family of the op set (FC and its fused twin / QKV forms, GQA
  * attention, every row-wise epilogue op including Drop, Softmax and the three softmax losses,
@@ -41,6 +41,7 @@
 #include "tkm_attn.h"
 #include "tkm_codegen_internal.h"
 #include "tkm_gemm.h"
+#include "tkm_gemm_mfma.h"
 #include "tkm_hip.h"
 #include "tkm_plasma_internal.h"
 #include "tkm_prep_internal.h"
@@ -72,7 +73,12 @@ typedef struct {
     void *xhat;
     void *mask;
     float *lse;
+    /* an FC layer's three products: this build's kernels where they take the shape (own_*), else
+     * hipBLASLt (g_*) */
     tkm_gemm *g_fwd, *g_dw, *g_dx;
+    TkmGemmProblem p_fwd, p_dw, p_dx;
+    int own_fwd, own_dw, own_dx;
+    int dw_last;                        /* the last node of own_dw in the backward walk: enqueues the group */
     int dx_first;                       /* GEMM dX is the first writer of grad(in0): beta 0 */
 } rt_node;
 
@@ -95,9 +101,13 @@ struct TkmRuntime {
     tkm_runtime_opts opts;
     int dt, training;
     hipStream_t stream;
-    /* Training: the weight-gradient GEMMs run on `side` with their own workspace, forked from
-     * `stream` at each GEMM node of the backward walk and joined before the reductions. */
+    /* Training: the weight-gradient GEMMs run on `side` (hipBLASLt's with their own workspace),
+     * forked from `stream` in the backward walk and joined before the reductions.  This build's
+     * own are one launch (plan_dw_group). */
     hipStream_t side;
+    TkmGemmProblem *d_dw;
+    int n_dw, dw_tile;
+    long long dw_tiles;
     hipEvent_t ev_fork, ev_join;
     void *lt;
     void *gemm_ws, *gemm_ws_side;
@@ -573,13 +583,24 @@ static int plan_gemms(TkmRuntime *rt) {
         st->in_dim = K;
         st->out_dim = N;
         st->rows = rows;
-        if (tkm_gemm_create(&st->g_fwd, rt->lt, 0, 0, N, rows, K, N, K, N, ab, ab, 0.0f, TKM_GEMM_MAX_WS)) goto fail;
+        rt_tensor *t = &rt->tensors[st->t_w];
+        uint8_t *x = rt->arena + g->nodes[n->in0].out_offset, *y = rt->arena + n->out_offset;
+        st->p_fwd = (TkmGemmProblem){x, t->w16, y, rows, N, K, K, N, N, 0};
+        st->own_fwd = tkm_gemm_mfma_supported(&st->p_fwd, 0);
+        if (!st->own_fwd && tkm_gemm_create(&st->g_fwd, rt->lt, 0, 0, N, rows, K, N, K, N, ab, ab, 0.0f, TKM_GEMM_MAX_WS))
+            goto fail;
         if (ws < tkm_gemm_workspace(st->g_fwd)) ws = tkm_gemm_workspace(st->g_fwd);
         if (rt->training) {
-            if (tkm_gemm_create(&st->g_dw, rt->lt, 0, 1, N, K, rows, N, K, N, ab, TKM_GEMM_F32, 0.0f, TKM_GEMM_MAX_WS))
+            uint8_t *dx = rt->grad_arena + g->nodes[n->in0].out_offset, *dy = rt->grad_arena + n->out_offset;
+            st->p_dw = (TkmGemmProblem){x, dy, t->grad, K, N, rows, K, N, N, 0};
+            st->p_dx = (TkmGemmProblem){dy, t->w16, dx, rows, K, N, N, N, K, 0};
+            st->own_dw = tkm_gemm_mfma_supported(&st->p_dw, 1);
+            st->own_dx = tkm_gemm_mfma_supported(&st->p_dx, 0);
+            if (!st->own_dw && tkm_gemm_create(&st->g_dw, rt->lt, 0, 1, N, K, rows, N, K, N, ab, TKM_GEMM_F32, 0.0f,
+                                               TKM_GEMM_MAX_WS))
                 goto fail;
-            if (tkm_gemm_create(&st->g_dx, rt->lt, 1, 0, K, rows, N, N, N, K, ab, ab, st->dx_first ? 0.0f : 1.0f,
-                                TKM_GEMM_MAX_WS))
+            if (!st->own_dx && tkm_gemm_create(&st->g_dx, rt->lt, 1, 0, K, rows, N, N, N, K, ab, ab,
+                                               st->dx_first ? 0.0f : 1.0f, TKM_GEMM_MAX_WS))
                 goto fail;
             if (ws < tkm_gemm_workspace(st->g_dw)) ws = tkm_gemm_workspace(st->g_dw);
             if (ws < tkm_gemm_workspace(st->g_dx)) ws = tkm_gemm_workspace(st->g_dx);
@@ -594,6 +615,38 @@ static int plan_gemms(TkmRuntime *rt) {
     if (ws && !HIP_OK(hipMalloc(&rt->gemm_ws, ws))) return 0;
     if (ws && rt->training && !HIP_OK(hipMalloc(&rt->gemm_ws_side, ws))) return 0;
     return 1;
+}
+
+/* The weight gradients of all GEMM nodes the kernels take, as one launch at the last of them in the
+ * backward walk.  Launched node by node (on `side`, next to the dX chain) each has too few tiles for
+ * the chip, and its workgroups' LDS keeps the chain's GEMMs off their CUs: config 4's step took
+ * 2978 us with six launches beside the chain, 2910 with one at its end.  Tile size by the total:
+ * 256x128 reads LDS least per MFMA but needs some 4 tiles a CU (2910 against 2952 us there), 64x64
+ * fills the chip for small models. */
+static int plan_dw_group(TkmRuntime *rt) {
+    const TkmGraph *g = &rt->graph;
+    TkmGemmProblem *h = (TkmGemmProblem *)calloc((size_t)g->num_nodes, sizeof *h);
+    if (!h) return 0;
+    rt_node *last = NULL;
+    long long tiles = 0;
+    for (int i = g->num_nodes - 1; i >= 1; --i) {
+        rt_node *st = &rt->nodes[i];
+        if (!st->own_dw) continue;
+        h[rt->n_dw++] = st->p_dw;
+        tiles += tkm_gemm_mfma_tiles(&st->p_dw, TKM_GEMM_TILE_128x128);
+        last = st;
+    }
+    rt->dw_tile = tiles >= 1024 ? TKM_GEMM_TILE_256x128 : tiles >= 128 ? TKM_GEMM_TILE_128x128 : TKM_GEMM_TILE_64x64;
+    for (int k = 0; k < rt->n_dw; ++k) {
+        h[k].tile0 = rt->dw_tiles;
+        rt->dw_tiles += tkm_gemm_mfma_tiles(&h[k], rt->dw_tile);
+    }
+    if (last) last->dw_last = 1;
+    const int ok = rt->n_dw == 0 || (HIP_OK(hipMalloc((void **)&rt->d_dw, (size_t)rt->n_dw * sizeof *h)) &&
+                                     HIP_OK(hipMemcpy(rt->d_dw, h, (size_t)rt->n_dw * sizeof *h,
+                                                      hipMemcpyHostToDevice)));
+    free(h);
+    return ok;
 }
 
 static int plan_groups(TkmRuntime *rt) {
@@ -779,7 +832,7 @@ TkmRuntime *tkm_runtime_ignite_ex(const TkmGraph *g, const char *src, const tkm_
         *rt->h_pin_lr = 1e-3f;
     }
     if (!alloc_params(rt) || !alloc_saves(rt) || !plan_groups(rt) || !plan_grad_writes(rt) || !plan_gemms(rt) ||
-        (rt->training && !plan_reductions(rt)))
+        (rt->training && (!plan_dw_group(rt) || !plan_reductions(rt))))
         goto fail;
     free(own_src);
     if (opts.verbose)
@@ -937,8 +990,12 @@ static void forward_pass(TkmRuntime *rt, int is_eval, int valid_examples) {
         void *in = act(rt, n->in0), *out = act(rt, i);
         const int rows = (int)rows_of(g, n);
         if (is_gemm(n->op)) {
-            note(rt, tkm_gemm_run(st->g_fwd, rt->tensors[st->t_w].w16, in, out, rt->gemm_ws, rt->gemm_ws_bytes,
-                                  rt->stream), "GEMM forward");
+            if (st->own_fwd)
+                note(rt, tkm_gemm_mfma_run(&st->p_fwd, 0, rt->dt == TKM_ATTN_BF16, TKM_GEMM_TILE_AUTO, 0, rt->stream),
+                     "GEMM forward");
+            else
+                note(rt, tkm_gemm_run(st->g_fwd, rt->tensors[st->t_w].w16, in, out, rt->gemm_ws, rt->gemm_ws_bytes,
+                                      rt->stream), "GEMM forward");
         } else if (n->op == OP_GQA_ATTN) {
             note(rt, tkm_attn_fwd(in, out, st->lse, NULL, B, n->H * n->W, n->q_heads, n->kv_heads, n->head_dim,
                                   attn_scale(n->head_dim), n->causal ? 1 : 0, rt->dt, rt->stream),
@@ -982,14 +1039,23 @@ static void record_step(TkmRuntime *rt, int clear_loss) {
         rt_node *st = &rt->nodes[i];
         void *in_act = act(rt, n->in0), *out_act = act(rt, i), *dout = grd(rt, i), *din = grd(rt, n->in0);
         if (is_gemm(n->op)) {
-            /* dW on the side stream: its inputs (this node's gradient, complete once every
-             * consumer's backward ran, and the saved input activation) are never written again
-             * in the step, and only SGD reads its output */
+            /* dW on the side stream, at once or with the group: its inputs (this node's gradient,
+             * complete once every consumer's backward ran, and the saved input activation) are never
+             * written again in the step, and only SGD reads its output */
             rt_tensor *t = &rt->tensors[st->t_w];
-            depend(rt, rt->side, rt->stream, rt->ev_fork);
-            note(rt, tkm_gemm_run(st->g_dw, dout, in_act, t->grad, rt->gemm_ws_side, rt->gemm_ws_bytes, rt->side),
-                 "GEMM dW");
-            note(rt, tkm_gemm_run(st->g_dx, t->w16, dout, din, rt->gemm_ws, rt->gemm_ws_bytes, rt->stream), "GEMM dX");
+            if (!st->own_dw || st->dw_last) depend(rt, rt->side, rt->stream, rt->ev_fork);
+            if (!st->own_dw)
+                note(rt, tkm_gemm_run(st->g_dw, dout, in_act, t->grad, rt->gemm_ws_side, rt->gemm_ws_bytes, rt->side),
+                     "GEMM dW");
+            if (st->dw_last)
+                note(rt, tkm_gemm_mfma_group(rt->d_dw, rt->n_dw, rt->dw_tiles, rt->dt == TKM_ATTN_BF16, rt->dw_tile,
+                                             rt->side), "GEMM dW group");
+            if (st->own_dx)
+                note(rt, tkm_gemm_mfma_run(&st->p_dx, 1, rt->dt == TKM_ATTN_BF16, TKM_GEMM_TILE_AUTO, !st->dx_first,
+                                           rt->stream), "GEMM dX");
+            else
+                note(rt, tkm_gemm_run(st->g_dx, t->w16, dout, din, rt->gemm_ws, rt->gemm_ws_bytes, rt->stream),
+                     "GEMM dX");
         } else if (n->op == OP_GQA_ATTN) {
             note(rt, tkm_attn_bwd(in_act, out_act, dout, st->lse, din, NULL, B, n->H * n->W, n->q_heads, n->kv_heads,
                                   n->head_dim, attn_scale(n->head_dim), n->causal ? 1 : 0, rt->dt, rt->attn_ws,
@@ -1642,6 +1708,7 @@ static void free_runtime(TkmRuntime *rt) {
     hipFree(rt->attn_ws);
     hipFree(rt->part_ws);
     hipFree(rt->d_red);
+    hipFree(rt->d_dw);
     hipFree(rt->gemm_ws);
     hipFree(rt->gemm_ws_side);
     hipFree(rt->param_block);
