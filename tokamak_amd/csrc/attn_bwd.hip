@@ -91,14 +91,13 @@ __global__ __launch_bounds__(256) void fa_bwd_delta_kernel(const uint16_t* __res
 //   dV^T += dO^T P,  dK^T += Q^T dS the P / dS accumulators are the B operands in place,
 //                                  dO^T and Q^T come from transposed LDS reads
 // dK (times scale) and dV are written once; no atomics.
-// KSPLIT = 2 (small grids): two groups of NW waves over the same keys; group g walks every
-// other query tile of the key block's list through its own buffers (its waves load the same
-// K; group 0 moves the V rows both read), and group 1 adds its dK and dV accumulators into
-// group 0's through LDS before group 0 writes them.  NW = 4: blocks of 128 keys (one
-// workgroup of 8 waves per CU).  NW = 2 (causal): blocks of 64 keys, two workgroups of 4 waves
-// per CU, numbered so that the workgroups the dispatcher puts on one CU (blocks i and
-// i + grid/2) pair a heavy (early) key block with a light one.
-template <int D, int DT, int KSPLIT, int NW = 4>
+// KSPLIT > 1 (small grids): KSPLIT groups of NW waves over the same keys; group g walks every
+// KSPLIT-th query tile of the key block's list through its own buffers (its waves load the same
+// K; group 0 moves the V rows all read), and the groups' dK and dV accumulators are added through LDS
+// before group 0 writes them.  Blocks have 32 NW keys; with NW = 2 and causal they are numbered so that
+// the workgroups the dispatcher puts on one CU (blocks i and i + grid/2) pair a heavy (early) key
+// block with a light one.  attn_launch.h (pick_keys_form) has the choice and its measurements.
+template <int D, int DT, int KSPLIT, int NW>
 __global__ __launch_bounds__(64 * NW * KSPLIT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ dout,
                         const float* __restrict__ lse, const float* __restrict__ delta,
@@ -159,7 +158,7 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
                 for (int i = 0; i < 32 / RPI; ++i) {
                     const int r = i * RPI + lane / CPR;
                     dma16(rv, &sV[wave][i * RPI * ROWB],
-                          (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4));
+                          (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4), i == 0);
                 }
             }
         }
@@ -180,8 +179,8 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
             for (int i = 0; i < NI; ++i) {
                 const int r0 = (wave * NI + i) * RPI, r = r0 + dma_r;
                 const uint32_t sw = (uint32_t)((dma_p ^ swz<D>(r)) << 4);
-                dma16(rq, &smem[grp][buf][0][r0 * ROWB], (uint32_t)r * ldb + sw);
-                dma16(ro, &smem[grp][buf][1][r0 * ROWB], (uint32_t)r * ldob + sw);
+                dma16(rq, &smem[grp][buf][0][r0 * ROWB], (uint32_t)r * ldb + sw, i == 0);
+                dma16(ro, &smem[grp][buf][1][r0 * ROWB], (uint32_t)r * ldob + sw, i == 0);
             }
             if (wave == 0) {
                 const size_t li = ((size_t)b * Hq + h) * S + qr0;
@@ -285,32 +284,37 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
         }
     }
 
-    if constexpr (KSPLIT == 2) {
-        // Group 1's dK^T then dV^T accumulators into group 0's, through the Q/dO buffers (free
-        // once the last iteration ended with every DMA done and a barrier): element r of block
-        // db of wave w's lane at float ((db*16 + r)*NW + w)*64 + lane.
+    if constexpr (KSPLIT > 1) {
+        // The groups' dK^T then dV^T accumulators, added pairwise (group h + g into g, h halving) through the
+        // Q/dO buffers (free once the last iteration ended with every DMA done and a barrier): element r
+        // of block db of wave w's lane, handed over by group h + g, at float (((g*NDB + db)*16 + r)*NW + w)*64 + lane.
         float* xs = reinterpret_cast<float*>(&smem[0][0][0][0]);
-        static_assert(NDB * 16 * NW * 64 * 4 <= (int)sizeof(smem), "one accumulator set fits the buffers");
-        auto at = [&](int db, int r) -> float& { return xs[((db * 16 + r) * NW + wave) * 64 + lane]; };
+        static_assert(KSPLIT / 2 * NDB * 16 * NW * 64 * 4 <= (int)sizeof(smem), "the accumulator sets fit the buffers");
 #pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
-            f32x16(&acc)[NDB] = pass ? dv : dk;
-            if (grp == 1) {
+        for (int h = KSPLIT / 2; h > 0; h /= 2) {
+            auto at = [&](int db, int r) -> float& {
+                return xs[((((grp & (h - 1)) * NDB + db) * 16 + r) * NW + wave) * 64 + lane];
+            };
 #pragma unroll
-                for (int db = 0; db < NDB; ++db)
+            for (int pass = 0; pass < 2; ++pass) {
+                f32x16(&acc)[NDB] = pass ? dv : dk;
+                if (grp >= h && grp < 2 * h) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) at(db, r) = acc[db][r];
+                    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) at(db, r) = acc[db][r];
+                }
+                __syncthreads();
+                if (grp < h) {
+#pragma unroll
+                    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) acc[db][r] += at(db, r);
+                }
+                __syncthreads();
             }
-            __syncthreads();
-            if (grp == 0) {
-#pragma unroll
-                for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[db][r] += at(db, r);
-            }
-            __syncthreads();
         }
-        if (grp == 1) return;
+        if (grp > 0) return;
     }
 
     // dK^T (scaled), dV^T: lane holds key = kw0 + l32, d = db*32 + g4*8 + hi*4 + 0..3.
@@ -341,12 +345,9 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
 //   dS^T = P^T (dP^T - D),  dQ^T += K^T dS^T  (K^T from transposed LDS reads)
 // WD: D of the wave's rows is computed here (fp32 sum of O * dO over the lane pair that holds
 // the row) and written to delta instead of read from it.
-// KSPLIT = 2, NW = 2 (causal D = 64, small grids): blocks of 64 queries, two groups of two
-// waves over the same rows, group g walking its half of the key tiles through its own
-// buffers (both form D from the O rows; group 0 writes it); group 1 adds its dQ accumulators
-// into group 0's through LDS.  Two workgroups per CU, numbered so that blocks i and
-// i + grid/2 pair a heavy (late) query block with a light one.
-template <int D, int DT, bool WD, int KSPLIT = 1, int NW = 4>
+// KSPLIT, NW and BN as the forward's: the groups each walk their part of the key tiles (all form D
+// from the O rows; group 0 writes it) and their dQ accumulators are added through LDS.
+template <int D, int DT, bool WD, int KSPLIT, int NW, int BN>
 __global__ __launch_bounds__(64 * NW * KSPLIT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ o,
                       const uint16_t* __restrict__ dout, const float* __restrict__ lse,
@@ -354,7 +355,7 @@ void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restri
                       uint16_t* __restrict__ dqkv,
                       const int32_t* __restrict__ kv_len, int B, int S, int Hq, int Hkv,
                       float scale, float sl2, int causal, int n_qblk) {
-    constexpr int BM = 32 * NW, BN = 64;
+    constexpr int BM = 32 * NW;
     constexpr int KS = D / 16, NKB = BN / 32, NDB = D / 32, PKS = BN / 16;
     constexpr int ROWB = D * 2, CPR = D / 8, TILEB = BN * ROWB;
     constexpr int RPI = 64 / CPR, NI = BN / RPI / NW;
@@ -429,8 +430,8 @@ void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restri
     if (causal) kv_end = min(kv_end, qblk * BM + BM);
     const int ntiles = (kv_end + BN - 1) / BN;
     // this group's tiles [tb, te); every group runs nit iterations (barriers stay matched)
-    const int nit = KSPLIT == 2 ? (ntiles + 1) / 2 : ntiles;
-    const int tb = grp == 0 ? 0 : nit, te = grp == 0 ? nit : ntiles;
+    const int nit = (ntiles + KSPLIT - 1) / KSPLIT;
+    const int tb = grp * nit, te = min(tb + nit, ntiles);
 
     const int dma_r = lane / CPR, dma_p = lane % CPR;
     auto issue = [&](int t, int buf) __attribute__((always_inline)) {
@@ -442,8 +443,8 @@ void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restri
         for (int i = 0; i < NI; ++i) {
             const int r0 = (wave * NI + i) * RPI, r = r0 + dma_r;
             const uint32_t voff = (uint32_t)r * ldb + (uint32_t)((dma_p ^ swz<D>(r)) << 4);
-            dma16(rk, &smem[grp][buf][0][r0 * ROWB], voff);
-            dma16(rv, &smem[grp][buf][1][r0 * ROWB], voff);
+            dma16(rk, &smem[grp][buf][0][r0 * ROWB], voff, i == 0);
+            dma16(rv, &smem[grp][buf][1][r0 * ROWB], voff, i == 0);
         }
     };
     const int fk = swz<D>(l32);
@@ -528,27 +529,31 @@ void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restri
         __syncthreads();
     }
 
-    if constexpr (KSPLIT == 2) {
-        // Group 1's dQ^T accumulators into group 0's through the K/V buffers (free after the
-        // loop's last barrier): element r of block db of wave w's lane at float
-        // ((db*16 + r)*NW + w)*64 + lane.
+    if constexpr (KSPLIT > 1) {
+        // The groups' dQ^T accumulators, added pairwise (group h + g into g, h halving) through the K/V buffers
+        // (free after the loop's last barrier), laid out as the dK/dV kernel's.
         float* xs = reinterpret_cast<float*>(&smem[0][0][0][0]);
-        static_assert(NDB * 16 * NW * 64 * 4 <= (int)sizeof(smem), "one accumulator set fits the buffers");
-        auto at = [&](int db, int r) -> float& { return xs[((db * 16 + r) * NW + wave) * 64 + lane]; };
-        if (grp == 1) {
+        static_assert(KSPLIT / 2 * NDB * 16 * NW * 64 * 4 <= (int)sizeof(smem), "the accumulator sets fit the buffers");
 #pragma unroll
-            for (int db = 0; db < NDB; ++db)
+        for (int h = KSPLIT / 2; h > 0; h /= 2) {
+            auto at = [&](int db, int r) -> float& {
+                return xs[((((grp & (h - 1)) * NDB + db) * 16 + r) * NW + wave) * 64 + lane];
+            };
+            if (grp >= h && grp < 2 * h) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) at(db, r) = dq[db][r];
+                for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) at(db, r) = dq[db][r];
+            }
+            __syncthreads();
+            if (grp < h) {
+#pragma unroll
+                for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) dq[db][r] += at(db, r);
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        if (grp == 0) {
-#pragma unroll
-            for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) dq[db][r] += at(db, r);
-        }
-        __syncthreads();
     }
 
     // dQ (times scale) leaves through LDS: a lane holds query q, d = db*32 + g4*8 + hi*4 + 0..3;
@@ -589,85 +594,59 @@ static int launch_delta_t(const BwdArgs& a) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-static int compute_units_bwd() {
-    static int cached[64];
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-    if (cached[dev] <= 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-        cached[dev] = n;
-    }
-    return cached[dev];
+template <int D, int DT, int KSPLIT, int NW>
+static int launch_dkdv_v(const BwdArgs& a) {
+    const int n_kblk = (a.S + 32 * NW - 1) / (32 * NW);
+    hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, DT, KSPLIT, NW>), dim3((unsigned)((long long)a.B * a.Hkv * n_kblk)),
+                       dim3(64 * NW * KSPLIT), 0, (hipStream_t)a.stream, (const uint16_t*)a.qkv,
+                       (const uint16_t*)a.dout, a.lse, (const float*)a.delta, (uint16_t*)a.dqkv, a.kv_len, a.B, a.S,
+                       a.Hq, a.Hkv, a.scale, a.scale * 1.4426950408889634f, a.causal);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int D, int DT>
-static int launch_dkdv_t(const BwdArgs& a) {
-    constexpr int BN = 128;
-    const int n_kblk = (a.S + BN - 1) / BN;
-    const long long n_wg = (long long)a.B * a.Hkv * n_kblk;
-    dim3 grid((unsigned)n_wg);
-    // At most one workgroup of 128 keys per CU: split each key block's query tiles over two
-    // groups of waves.  Causal D = 64: blocks of 64 keys instead, two workgroups per CU
-    // (2 x 48 KB of LDS) pairing heavy and light key blocks.
+static int launch_dkdv_t(const BwdArgs& a, HipForm form) {
     if constexpr (D == 64) {
-        if (n_wg <= compute_units_bwd() && a.causal) {
-            dim3 grid64((unsigned)((long long)a.B * a.Hkv * ((a.S + 63) / 64)));
-            hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, DT, 2, 2>), grid64, dim3(256), 0, (hipStream_t)a.stream,
-                               (const uint16_t*)a.qkv, (const uint16_t*)a.dout, a.lse, (const float*)a.delta,
-                               (uint16_t*)a.dqkv, a.kv_len, a.B, a.S, a.Hq, a.Hkv, a.scale,
-                               a.scale * 1.4426950408889634f, a.causal);
-            return hipGetLastError() == hipSuccess ? 0 : -1;
-        }
+        if (form == kForm2x2) return launch_dkdv_v<D, DT, 2, 2>(a);
+        if (form == kForm8x1) return launch_dkdv_v<D, DT, 8, 1>(a);
+    } else {
+        if (form == kForm2x4) return launch_dkdv_v<D, DT, 2, 4>(a);
     }
-    if (n_wg <= compute_units_bwd())
-        hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, DT, 2>), grid, dim3(512), 0, (hipStream_t)a.stream,
-                           (const uint16_t*)a.qkv, (const uint16_t*)a.dout, a.lse, (const float*)a.delta,
-                           (uint16_t*)a.dqkv, a.kv_len, a.B, a.S, a.Hq, a.Hkv, a.scale,
-                           a.scale * 1.4426950408889634f, a.causal);
-    else
-        hipLaunchKernelGGL((fa_bwd_dkdv_kernel<D, DT, 1>), grid, dim3(256), 0, (hipStream_t)a.stream,
-                           (const uint16_t*)a.qkv, (const uint16_t*)a.dout, a.lse, (const float*)a.delta,
-                           (uint16_t*)a.dqkv, a.kv_len, a.B, a.S, a.Hq, a.Hkv, a.scale,
-                           a.scale * 1.4426950408889634f, a.causal);
+    if (form == kForm4x1) return launch_dkdv_v<D, DT, 4, 1>(a);
+    return launch_dkdv_v<D, DT, 1, 4>(a);
+}
+
+template <int D, int DT, bool WD, int KSPLIT, int NW, int BN>
+static int launch_dq_v(const BwdArgs& a) {
+    const int n_qblk = (a.S + 32 * NW - 1) / (32 * NW);
+    hipLaunchKernelGGL((fa_bwd_dq_kernel<D, DT, WD, KSPLIT, NW, BN>), dim3((unsigned)((long long)a.B * a.Hq * n_qblk)),
+                       dim3(64 * NW * KSPLIT), 0, (hipStream_t)a.stream, (const uint16_t*)a.qkv, (const uint16_t*)a.o,
+                       (const uint16_t*)a.dout, a.lse, a.delta, a.ld, (uint16_t*)a.dqkv, a.kv_len, a.B, a.S, a.Hq,
+                       a.Hkv, a.scale, a.scale * 1.4426950408889634f, a.causal, n_qblk);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int D, int DT, bool WD>
-static int launch_dq_t(const BwdArgs& a) {
-    constexpr int BM = 128;
-    const int n_qblk = (a.S + BM - 1) / BM;
-    // Causal D = 64 with at most one 128-row block per CU: 64-row blocks over two groups of
-    // two waves (each walks half the key tiles), two workgroups per CU pairing heavy and light.
+static int launch_dq_t(const BwdArgs& a, HipForm form) {
+    if (form == kForm4x1) return launch_dq_v<D, DT, WD, 4, 1, 32>(a);
+    if (form == kForm4x2) return launch_dq_v<D, DT, WD, 4, 2, D == 64 ? 64 : 32>(a);
     if constexpr (D == 64) {
-        if (a.causal && (long long)a.B * a.Hq * n_qblk <= compute_units_bwd()) {
-            const int n_qblk64 = (a.S + 63) / 64;
-            hipLaunchKernelGGL((fa_bwd_dq_kernel<D, DT, WD, 2, 2>), dim3((unsigned)(a.B * a.Hq * n_qblk64)),
-                               dim3(256), 0, (hipStream_t)a.stream,
-                               (const uint16_t*)a.qkv, (const uint16_t*)a.o, (const uint16_t*)a.dout, a.lse,
-                               a.delta, a.ld, (uint16_t*)a.dqkv, a.kv_len, a.B, a.S, a.Hq, a.Hkv, a.scale,
-                               a.scale * 1.4426950408889634f, a.causal, n_qblk64);
-            return hipGetLastError() == hipSuccess ? 0 : -1;
-        }
+        if (form == kForm2x2) return launch_dq_v<D, DT, WD, 2, 2, 64>(a);
     }
-    dim3 grid((unsigned)(a.B * a.Hq * n_qblk)), block(256);
-    hipLaunchKernelGGL((fa_bwd_dq_kernel<D, DT, WD>), grid, block, 0, (hipStream_t)a.stream,
-                       (const uint16_t*)a.qkv, (const uint16_t*)a.o, (const uint16_t*)a.dout, a.lse,
-                       a.delta, a.ld, (uint16_t*)a.dqkv, a.kv_len, a.B, a.S, a.Hq, a.Hkv, a.scale,
-                       a.scale * 1.4426950408889634f, a.causal, n_qblk);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
+    if (form == kForm2x4) return launch_dq_v<D, DT, WD, 2, 4, 64>(a);
+    return launch_dq_v<D, DT, WD, 1, 4, 64>(a);
 }
 template <int D, int DT>
-static int launch_dq_read_t(const BwdArgs& a) { return launch_dq_t<D, DT, false>(a); }
+static int launch_dq_read_t(const BwdArgs& a, HipForm form) { return launch_dq_t<D, DT, false>(a, form); }
 template <int D, int DT>
-static int launch_dq_write_t(const BwdArgs& a) { return launch_dq_t<D, DT, true>(a); }
+static int launch_dq_write_t(const BwdArgs& a, HipForm form) { return launch_dq_t<D, DT, true>(a, form); }
 
-#define TKM_DISPATCH(FN, a)                                                                 \
-    ((a).D == 128 ? ((a).dtype == DT_F16 ? FN<128, DT_F16>(a) : FN<128, DT_BF16>(a))        \
-                  : ((a).dtype == DT_F16 ? FN<64, DT_F16>(a) : FN<64, DT_BF16>(a)))
+#define TKM_DISPATCH(FN, a, ...)                                                                              \
+    ((a).D == 128 ? ((a).dtype == DT_F16 ? FN<128, DT_F16>(a __VA_OPT__(, ) __VA_ARGS__)                     \
+                                         : FN<128, DT_BF16>(a __VA_OPT__(, ) __VA_ARGS__))                   \
+                  : ((a).dtype == DT_F16 ? FN<64, DT_F16>(a __VA_OPT__(, ) __VA_ARGS__)                      \
+                                         : FN<64, DT_BF16>(a __VA_OPT__(, ) __VA_ARGS__)))
 
-// Each stage tries its assembly kernel first (D = 128 fp16); 1 from it means "not handled
-// there" and selects the HIP kernel, any other status is final.
 static int settle(int r, unsigned asm_bit) {
     if (r == 0) note_kernels(asm_bit);
     return r;
@@ -677,23 +656,33 @@ int launch_bwd_delta(const BwdArgs& a) {
     note_kernels(kDeltaHip);
     return TKM_DISPATCH(launch_delta_t, a);
 }
+// Each stage that the rule gives to an assembly kernel falls to the HIP kernel's plain forms where
+// that one declines the shape (1); any other status of it is final.
 int launch_bwd_dkdv(const BwdArgs& a) {
-    const int r = launch_bwd_dkdv_asm(a);
-    if (r != 1) return settle(r, kDkdvAsm);
+    const int n = compute_units();
+    const long long k = (long long)a.B * a.Hkv * ((a.S + 127) / 128);
+    HipForm form = pick_keys_form(a.D, k, a.S, a.Hq / a.Hkv, a.causal != 0, n);
+    if (form == kFormAsm) {
+        const int r = launch_bwd_dkdv_asm(a);
+        if (r != 1) return settle(r, kDkdvAsm);
+        form = k <= n ? kForm2x4 : kForm1x4;
+    }
     note_kernels(kDkdvHip);
-    return TKM_DISPATCH(launch_dkdv_t, a);
+    return TKM_DISPATCH(launch_dkdv_t, a, form);
 }
-int launch_bwd_dq(const BwdArgs& a) {
-    const int r = launch_bwd_dq_asm(a, false);
-    if (r != 1) return settle(r, kDqAsm);
+static int launch_dq(const BwdArgs& a, bool write_d) {
+    const int n = compute_units();
+    const long long q = (long long)a.B * a.Hq * ((a.S + 127) / 128);
+    HipForm form = pick_rows_form(a.D, true, q, a.S, a.causal != 0, n);
+    if (form == kFormAsm) {
+        const int r = launch_bwd_dq_asm(a, write_d);
+        if (r != 1) return settle(r, kDqAsm);
+        form = q <= n ? kForm2x4 : kForm1x4;
+    }
     note_kernels(kDqHip);
-    return TKM_DISPATCH(launch_dq_read_t, a);
+    return write_d ? TKM_DISPATCH(launch_dq_write_t, a, form) : TKM_DISPATCH(launch_dq_read_t, a, form);
 }
-int launch_bwd_dq_delta(const BwdArgs& a) {
-    const int r = launch_bwd_dq_asm(a, true);
-    if (r != 1) return settle(r, kDqAsm);
-    note_kernels(kDqHip);
-    return TKM_DISPATCH(launch_dq_write_t, a);
-}
+int launch_bwd_dq(const BwdArgs& a) { return launch_dq(a, false); }
+int launch_bwd_dq_delta(const BwdArgs& a) { return launch_dq(a, true); }
 
 }  // namespace tkm

@@ -62,18 +62,6 @@ __device__ __forceinline__ uint32_t pack2(float x, float y) {
     }
 }
 
-// Sum of the two 16-bit values in w, accumulated in fp32.
-template <int DT>
-__device__ __forceinline__ float dot2_ones(uint32_t w, float acc) {
-    if constexpr (DT == DT_F16) {
-        const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w), one, acc, false);
-    } else {
-        const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), one, acc, false);
-    }
-}
-
 // bf16 keeps 8 significant bits, too few for the probabilities P and dS that feed the
 // second GEMM of each pair at the stated tolerance.  In bf16 mode they are therefore split
 // into hi = bf16(x) and lo = bf16(x - hi) and both halves go through the MFMA (same A
@@ -172,11 +160,13 @@ __device__ __forceinline__ void sched_steady() {
 // Buffer resources and HBM -> LDS DMA.
 // A raw buffer resource covering `bytes` bytes from `base`: loads at offsets beyond it
 // return zero, which is how partial tiles (rows >= S or >= kv_len) are zero-filled.
-// Both arguments must be wave-uniform; readfirstlane makes that explicit so the descriptor
-// lives in SGPRs (a VGPR descriptor would need a waterfall loop around every load).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0,
-                                             __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+// Both arguments must be wave-uniform; readfirstlane makes that explicit, so the four words are
+// scalars (also for the inline assembly below).
+__device__ __forceinline__ u32x4 make_rsrc(const void* base, uint32_t bytes) {
+    const uint64_t p = (uint64_t)base;
+    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((p >> 32) & 0xffffu)),
+                 (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
 }
 // Bytes a descriptor over `rows` rows of `pitch` bytes needs when lanes touch only the first
 // `width` bytes of each row: it ends at the last row's last touched byte, never at the row's
@@ -185,16 +175,33 @@ __device__ __forceinline__ uint32_t rows_bytes(int rows, uint32_t pitch, uint32_
     return rows > 0 ? (uint32_t)(rows - 1) * pitch + width : 0u;
 }
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-// 16 bytes per lane from rsrc+voffset into LDS at lds + 16*lane (lds is wave-uniform).
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, const void* lds, uint32_t voffset) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds, 16, voffset, 0, 0, 0);
+// HBM -> LDS DMA: 16 (4) bytes per lane from rsrc + voffset to LDS at lds + 16 (4) * lane (lds is
+// wave-uniform).  In inline assembly, because the compiler follows the DMA builtin's LDS writes
+// conservatively: before the first transposed read (ld_lds_tr) after one it waits for every load in
+// flight, which ends the prefetch of the next tile in the middle of the current one.  The asm writes no
+// register; a tile's requests are awaited by wait_dma (or a counted wait) and a barrier before its
+// first read.  first: the descriptor may have just been written by a VALU lane read, which a buffer
+// access may follow only after 5 wait states; otherwise 1, between the write of m0 and its use.
+__device__ __forceinline__ void dma16(u32x4 r, const void* lds, uint32_t voffset, bool first = true) {
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
+    if (first)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     : : "s"(at), "v"(voffset), "s"(r));
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     : : "s"(at), "v"(voffset), "s"(r));
 }
-// Wait until every memory operation of this wave, LDS DMA included, has completed.
-// 4 bytes per lane from rsrc+voffset into LDS at lds + 4*lane.
-__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, const void* lds, uint32_t voffset) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)lds, 4, voffset, 0, 0, 0);
+__device__ __forceinline__ void dma4(u32x4 r, const void* lds, uint32_t voffset) {
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 : : "s"(at), "v"(voffset), "s"(r));
 }
-__device__ __forceinline__ void wait_dma() { __builtin_amdgcn_s_waitcnt(0); }
+// Wait until every memory operation of this wave, LDS DMA included, has completed.  The builtin, so
+// that the compiler knows its own loads done too and adds no wait for them inside the tile loop.
+__device__ __forceinline__ void wait_dma() {
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" : : : "memory");
+}
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 // ds_read_b64_tr_b16: within each group of 16 lanes, lane i receives element i%4 of the

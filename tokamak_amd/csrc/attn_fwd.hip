@@ -17,8 +17,7 @@
 // Per tile and wave:
 //   S^T = K Q^T        32 keys x 32 queries per MFMA block; lane = query row.
 //   P^T = exp2(S^T * scale*log2e - m) with m the row offset (log2 units, below); the row sum
-//                      is an fp32 dot of the rounded P per lane, lane halves combined at the
-//                      end.
+//                      is the lane's fp32 sum of P, lane halves combined at the end.
 //   O^T += V^T P^T     the P^T accumulator, rounded to 16 bits, is the B operand in place;
 //                      V^T comes from the row-major V tile through ds_read_b64_tr_b16.
 //
@@ -32,8 +31,7 @@
 // fp32 (a scale folded into Q and rounded to 16 bits would move a score s by up to
 // |s|*2^-12, which trained attention logits turn into errors past the bars).  m starts as
 // the row max of the first tile and moves only when it must (a lazy online softmax): when a
-// later tile's packed P sum reaches fp16's largest value (a P past the fp16 range gives an
-// infinite sum), the wave raises m of its rows to max(m, the tile's row max), multiplies O and
+// later tile's P sum reaches fp16's largest value, the wave raises m of its rows to max(m, the tile's row max), multiplies O and
 // the row sums by 2^(m_old - m_new) and repeats the tile's exp2 before its PV product.
 // Causal: tiles above the diagonal are neither loaded nor computed, tiles crossing the
 // diagonal (or the kv_len / S edge) are masked, heaviest query blocks are launched first.
@@ -45,25 +43,25 @@
 
 namespace tkm {
 
-// A lane's packed P sum over a tile at or above this moves m (see softmax_next): fp16's
+// A lane's P sum over a tile at or above this moves m (see softmax_next): fp16's
 // largest finite value, so no P that reaches a PV product exceeds it, in either type.
 constexpr float P_SUM_MAX = 65504.0f;
 
-// KSPLIT = 2 (small grids): two groups of NW waves over the same query rows; group g walks its
-// own half of the block's key tiles through its own buffers, with its own m, and group 1 hands
-// (m, l, O) to group 0 through LDS at the end, which merges them (rescaling each side by
-// 2^(m_side - m)) and writes O and LSE.  The heaviest causal block then walks half its tiles.
-// NW = 4: blocks of 128 rows (one workgroup of 8 waves per CU).  NW = 2 (causal): blocks of 64
-// rows, two workgroups of 4 waves per CU, numbered so that the workgroups the dispatcher puts
-// on one CU (blocks i and i + grid/2) pair a heavy block with a light one.
-template <int D, int DT, int QB, int KSPLIT, int NW = 4>
+// KSPLIT > 1 (small grids): KSPLIT groups of NW waves over the same query rows; group g walks its
+// own part of the block's key tiles through its own buffers, with its own m, and the groups' (m, l, O)
+// are merged through LDS at the end (rescaling each side by 2^(m_side - m)).  The heaviest causal
+// block then walks 1/KSPLIT of its tiles.  Blocks have 32 NW rows; with NW = 2 and causal they
+// are numbered so that the workgroups the dispatcher puts on one CU (blocks i and i + grid/2) pair
+// a heavy block with a light one.  BN: keys per tile (32 where four groups' buffers of 64 would
+// not fit).  attn_launch.h (pick_rows_form) has the choice and its measurements.
+template <int D, int DT, int QB, int KSPLIT, int NW, int BN>
 __global__ __launch_bounds__(64 * NW * KSPLIT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
                    float* __restrict__ lse, const int32_t* __restrict__ kv_len, int B, int S,
                    int Hq, int Hkv, float sl2, int causal, int n_qblk) {
     constexpr bool SPL = Split<DT>::on;   // bf16: P as hi + lo
     constexpr int WR = 32 * QB;           // query rows per wave
-    constexpr int BM = NW * WR, BN = 64;
+    constexpr int BM = NW * WR;
     constexpr int KS = D / 16;    // k-steps over the head dim (S^T)
     constexpr int NKB = BN / 32;  // 32-key blocks per tile
     constexpr int NDB = D / 32;   // 32-wide head-dim blocks of O
@@ -120,8 +118,8 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
     // tiles [0, n_act) hold at least one key visible to this wave
     const int n_act = causal ? min(ntiles, (q0 + WR - 1) / BN + 1) : ntiles;
     // this group's tiles [tb, te); every group runs nit iterations (barriers stay matched)
-    const int nit = KSPLIT == 2 ? (ntiles + 1) / 2 : ntiles;
-    const int tb = grp == 0 ? 0 : nit, te = grp == 0 ? nit : ntiles;
+    const int nit = (ntiles + KSPLIT - 1) / KSPLIT;
+    const int tb = grp * nit, te = min(tb + nit, ntiles);
 
     // DMA of one tile (tensor 0 = K, 1 = V) into buffer buf: wave w moves rows
     // [w*NI*RPI, (w+1)*NI*RPI) of the BN-row tile.
@@ -134,7 +132,7 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
         for (int i = 0; i < NI; ++i) {
             const int r0 = (gw * NI + i) * RPI, row = r0 + dma_r;
             dma16(r, &smem[grp][tensor][buf][r0 * ROWB],
-                  (uint32_t)row * ldb + (uint32_t)((dma_p ^ swz<D>(row)) << 4));
+                  (uint32_t)row * ldb + (uint32_t)((dma_p ^ swz<D>(row)) << 4), i == 0);
         }
     };
 
@@ -206,7 +204,9 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
         }
     };
     // exp2 of the scores in set J (relative to mm[qb]), packed to 16 bits into P set J;
-    // lt[qb] = the lane's fp32 sum of the packed values.
+    // lt[qb] = the lane's sum of the fp32 values, as the assembly kernels and the reference's
+    // (tkm_gpu.cu:403) sum them: LSE is then within 1e-7 of 64 bits, against 2e-6 to 8e-6 with the
+    // sum of the packed values.
     auto stage_exp = [&](auto Jc, const float (&mm)[QB], float (&lt)[QB]) __attribute__((always_inline)) {
         constexpr int J = decltype(Jc)::value;
 #pragma unroll
@@ -225,12 +225,10 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
                         const u32x2 hl = pack_split_bf16(p0, p1);
                         pr[J][qb][ks][w] = hl[0];
                         plr[J][qb][ks][w] = hl[1];
-                        lt[qb] = dot2_ones<DT>(hl[1], dot2_ones<DT>(hl[0], lt[qb]));
                     } else {
-                        const uint32_t pw = pack2<DT>(p0, p1);
-                        pr[J][qb][ks][w] = pw;
-                        lt[qb] = dot2_ones<DT>(pw, lt[qb]);
+                        pr[J][qb][ks][w] = pack2<DT>(p0, p1);
                     }
+                    lt[qb] += p0 + p1;
                 }
             }
         }
@@ -275,8 +273,8 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
         }
         stage_exp(Jc, m, lsum);
     };
-    // Later tiles, against m.  A lane whose packed row sum of the tile reaches P_SUM_MAX (some
-    // P near or past fp16's range, where the fp16 pack gives an infinite sum) makes the wave
+    // Later tiles, against m.  A lane whose row sum of the tile reaches P_SUM_MAX (some P near or
+    // past fp16's range, where the fp16 pack gives infinity) makes the wave
     // raise m of its rows to max(m, the tile's row max), rescale O and the row sums by
     // 2^(m_old - m_new) (exactly 1 for rows whose m stays) and repeat the tile's exp2 and
     // packing, all before the tile's PV.  The bound holds for bf16 too: bf16 P would not
@@ -338,46 +336,55 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
         if (i + 1 < nit) iteration(I1{}, i + 1);
     }
 
-    if constexpr (KSPLIT == 2) {
-        // Group 1's m, partial row sums and O^T accumulators to group 0 (the buffers are free:
-        // the last iteration ended with every DMA done and a barrier).  Element j of the
-        // state of wave gw's lane sits at float (j*NW + gw)*64 + lane.
+    if constexpr (KSPLIT > 1) {
+        // The groups' m, partial row sums and O^T accumulators, merged pairwise (group h + g into g, h halving)
+        // through LDS (the buffers are free: the last iteration ended with every DMA done and a
+        // barrier).  Element j of the state group h + g hands over sits, for wave gw's lane, at float
+        // ((g*NV + j)*NW + gw)*64 + lane.
         constexpr int NV = QB * (2 + NDB * 16);
         float* xs = reinterpret_cast<float*>(&smem[0][0][0][0]);
-        static_assert(NV * NW * 64 * 4 <= (int)sizeof(smem), "merge state fits the tile buffers");
-        auto at = [&](int j) -> float& { return xs[(j * NW + gw) * 64 + lane]; };
-        if (grp == 1) {
+        static_assert(KSPLIT / 2 * NV * NW * 64 * 4 <= (int)sizeof(smem), "merge states fit the tile buffers");
 #pragma unroll
-            for (int qb = 0; qb < QB; ++qb) {
-                at(qb * (2 + NDB * 16)) = m[qb];
-                at(qb * (2 + NDB * 16) + 1) = lsum[qb];
+        for (int h = KSPLIT / 2; h > 0; h /= 2) {
+            auto at = [&](int j) -> float& { return xs[(((grp & (h - 1)) * NV + j) * NW + gw) * 64 + lane]; };
+            if (grp >= h && grp < 2 * h) {
 #pragma unroll
-                for (int db = 0; db < NDB; ++db)
+                for (int qb = 0; qb < QB; ++qb) {
+                    at(qb * (2 + NDB * 16)) = m[qb];
+                    at(qb * (2 + NDB * 16) + 1) = lsum[qb];
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) at(qb * (2 + NDB * 16) + 2 + db * 16 + r) = o[db][qb][r];
+                    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) at(qb * (2 + NDB * 16) + 2 + db * 16 + r) = o[db][qb][r];
+                }
             }
-        }
-        __syncthreads();
-        if (grp == 1) return;
+            __syncthreads();
+            if (grp < h) {
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb) {
-            const int base = qb * (2 + NDB * 16);
-            const float m1 = at(base), l1 = at(base + 1);
-            // a side without a visible key of the row (its row sum 0) takes no part
-            const float L0 = half_sum(lsum[qb]), L1 = half_sum(l1);
-            if (L1 > 0.f) {
-                const float mn = L0 > 0.f ? fmaxf(m[qb], m1) : m1;
-                const float a0 = L0 > 0.f ? fast_exp2(m[qb] - mn) : 0.f;
-                const float a1 = fast_exp2(m1 - mn);
-                lsum[qb] = lsum[qb] * a0 + l1 * a1;
+                for (int qb = 0; qb < QB; ++qb) {
+                    const int base = qb * (2 + NDB * 16);
+                    const float m1 = at(base), l1 = at(base + 1);
+                    // a side without a visible key of the row (its row sum 0) takes no part; one
+                    // whose sum is NaN does, so that a NaN score reaches O from either side
+                    const float L0 = half_sum(lsum[qb]), L1 = half_sum(l1);
+                    if (!(L1 <= 0.f)) {
+                        const bool own = !(L0 <= 0.f);
+                        const float mn = own ? fmaxf(m[qb], m1) : m1;
+                        const float a0 = own ? fast_exp2(m[qb] - mn) : 0.f;
+                        const float a1 = fast_exp2(m1 - mn);
+                        lsum[qb] = lsum[qb] * a0 + l1 * a1;
 #pragma unroll
-                for (int db = 0; db < NDB; ++db)
+                        for (int db = 0; db < NDB; ++db)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        o[db][qb][r] = o[db][qb][r] * a0 + at(base + 2 + db * 16 + r) * a1;
-                m[qb] = mn;
+                            for (int r = 0; r < 16; ++r)
+                                o[db][qb][r] = o[db][qb][r] * a0 + at(base + 2 + db * 16 + r) * a1;
+                        m[qb] = mn;
+                    }
+                }
             }
+            if (h > 1) __syncthreads();
         }
+        if (grp > 0) return;
     }
 
 #pragma unroll
@@ -402,8 +409,7 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
     }
 }
 
-// Compute units of the current device (cached per device; 0 if it cannot be read).
-static int compute_units() {
+int compute_units() {
     static int cached[64];
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
@@ -415,49 +421,43 @@ static int compute_units() {
     return cached[dev];
 }
 
-template <int D, int DT>
-static int launch_fwd_t(const FwdArgs& a) {
-    constexpr int QB = 1;  // 32-row blocks per wave
-    constexpr int BM = 128 * QB;
-    const int n_qblk = (a.S + BM - 1) / BM;
-    const long long n_wg = (long long)a.B * a.Hq * n_qblk;
-    dim3 grid((unsigned)n_wg);
-    // At most one workgroup of 128 rows per CU: split each block's keys over two groups of
-    // waves (the critical causal block walks half its tiles, and every SIMD holds two waves).
-    // Causal D = 64: blocks of 64 rows instead, two workgroups per CU (2 x 64 KB of LDS)
-    // pairing heavy and light blocks, so that no CU holds more than about the mean number of
-    // tiles.  (At D = 128 two such workgroups would need 256 KB of LDS.)
-    if constexpr (D == 64) {
-        if (n_wg <= compute_units() && a.causal) {
-            const int n_qblk64 = (a.S + 63) / 64;
-            dim3 grid64((unsigned)((long long)a.B * a.Hq * n_qblk64));
-            hipLaunchKernelGGL((fa_fwd_kernel<D, DT, QB, 2, 2>), grid64, dim3(256), 0, (hipStream_t)a.stream,
-                               (const uint16_t*)a.qkv, (uint16_t*)a.o, a.lse, a.kv_len, a.B, a.S, a.Hq,
-                               a.Hkv, a.scale * 1.4426950408889634f, a.causal, n_qblk64);
-            return hipGetLastError() == hipSuccess ? 0 : -1;
-        }
-    }
-    if (n_wg <= compute_units()) {
-        hipLaunchKernelGGL((fa_fwd_kernel<D, DT, QB, 2>), grid, dim3(512), 0, (hipStream_t)a.stream,
-                           (const uint16_t*)a.qkv, (uint16_t*)a.o, a.lse, a.kv_len, a.B, a.S, a.Hq,
-                           a.Hkv, a.scale * 1.4426950408889634f, a.causal, n_qblk);
-    } else {
-        hipLaunchKernelGGL((fa_fwd_kernel<D, DT, QB, 1>), grid, dim3(256), 0, (hipStream_t)a.stream,
-                           (const uint16_t*)a.qkv, (uint16_t*)a.o, a.lse, a.kv_len, a.B, a.S, a.Hq,
-                           a.Hkv, a.scale * 1.4426950408889634f, a.causal, n_qblk);
-    }
+template <int D, int DT, int KSPLIT, int NW, int BN>
+static int launch_fwd_v(const FwdArgs& a) {
+    const int n_qblk = (a.S + 32 * NW - 1) / (32 * NW);
+    hipLaunchKernelGGL((fa_fwd_kernel<D, DT, 1, KSPLIT, NW, BN>), dim3((unsigned)((long long)a.B * a.Hq * n_qblk)),
+                       dim3(64 * NW * KSPLIT), 0, (hipStream_t)a.stream, (const uint16_t*)a.qkv, (uint16_t*)a.o, a.lse,
+                       a.kv_len, a.B, a.S, a.Hq, a.Hkv, a.scale * 1.4426950408889634f, a.causal, n_qblk);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+template <int D, int DT>
+static int launch_fwd_t(const FwdArgs& a, HipForm form) {
+    // four groups' double buffers of 64-key tiles fit the LDS at D = 64 and two waves only
+    if (form == kForm4x1) return launch_fwd_v<D, DT, 4, 1, 32>(a);
+    if (form == kForm4x2) return launch_fwd_v<D, DT, 4, 2, D == 64 ? 64 : 32>(a);
+    if constexpr (D == 64) {
+        if (form == kForm2x2) return launch_fwd_v<D, DT, 2, 2, 64>(a);
+    }
+    if (form == kForm2x4) return launch_fwd_v<D, DT, 2, 4, 64>(a);
+    return launch_fwd_v<D, DT, 1, 4, 64>(a);
+}
+
 int launch_fwd(const FwdArgs& a) {
-    const int rc = launch_fwd_asm(a);  // D = 128 fp16 and bf16: hand-scheduled assembly kernels
-    if (rc != 1) {
-        if (rc == 0) note_kernels(kFwdAsm);
-        return rc;
+    const int n = compute_units();
+    const long long q = (long long)a.B * a.Hq * ((a.S + 127) / 128);
+    HipForm form = pick_rows_form(a.D, false, q, a.S, a.causal != 0, n);
+    if (form == kFormAsm) {
+        const int rc = launch_fwd_asm(a);  // D = 128 fp16 and bf16: hand-scheduled assembly kernels
+        if (rc != 1) {
+            if (rc == 0) note_kernels(kFwdAsm);
+            return rc;
+        }
+        form = q <= n ? kForm2x4 : kForm1x4;   // offsets past the assembly kernels' 32 bits
     }
     note_kernels(kFwdHip);
-    if (a.D == 128) return a.dtype == DT_F16 ? launch_fwd_t<128, DT_F16>(a) : launch_fwd_t<128, DT_BF16>(a);
-    return a.dtype == DT_F16 ? launch_fwd_t<64, DT_F16>(a) : launch_fwd_t<64, DT_BF16>(a);
+    if (a.D == 128)
+        return a.dtype == DT_F16 ? launch_fwd_t<128, DT_F16>(a, form) : launch_fwd_t<128, DT_BF16>(a, form);
+    return a.dtype == DT_F16 ? launch_fwd_t<64, DT_F16>(a, form) : launch_fwd_t<64, DT_BF16>(a, form);
 }
 
 }  // namespace tkm

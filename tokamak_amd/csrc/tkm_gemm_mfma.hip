@@ -15,9 +15,8 @@
 // the latency of the first loads and the fill of the chip by few tiles weigh as much as the matrix rate;
 // and the transposing reads deliver half the bytes per cycle, so dW (both operands NC) is bound by LDS
 // reads.  Hence several tile sizes (pick_tile), STAGES k-steps of LDS with STAGES - 1 in flight, a fixed
-// place for every LDS read and request between the MFMAs (in one burst they hold the wave's issue: dW
-// K 4096, N 8192: 65 -> 46 us), and the DMA issued from inline assembly (behind the DMA builtin the compiler
-// waits for every load in flight before each batch of transposed reads).
+// place for every LDS read and request between the MFMAs (in one burst they hold the wave's issue: dW of
+// 4096 rows, 512 x 8192: 65 -> 46 us).
 // Measured in bf16 at rows 4096, against hipBLASLt's first choice in the same training step:
 //   forward  N 1536, K 512 : 12.8 us (17.5)     dX  N 512, K 1536 : 12.1 us (24.5)
 //            N 512,  K 512 :  7.2 us (12.8)         N 512, K 512  :  6.9 us (10.4)
@@ -42,29 +41,9 @@ using namespace tkm;
 
 constexpr int BK = 64, KST = BK / 16;   // k of one step, its MFMA k-groups
 
-// Buffer descriptor as four scalar words (for inline assembly).
+// Descriptor of what is left of an operand (0 bytes or less: every request is out of range).
 __device__ __forceinline__ u32x4 desc(const char* base, long long bytes) {
-    const uint64_t p = (uint64_t)base;
-    const uint32_t n = bytes <= 0 ? 0u : (bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes);
-    return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
-                 (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((p >> 32) & 0xffffu)),
-                 (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
-}
-
-// 16 bytes per lane from descriptor + voff to LDS at lds + 16 * lane.  No register is written; the
-// compiler does not see the load, so each step waits for it explicitly (wait_step).
-// FIRST: the descriptor may have just been written by a VALU lane read, which a buffer access may
-// follow only after 5 wait states; otherwise one, between the write of m0 and its use.
-template <bool FIRST>
-__device__ __forceinline__ void dma_asm(u32x4 d, uint32_t lds, uint32_t voff) {
-    if constexpr (FIRST)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     :
-                     : "s"(lds), "v"(voff), "s"(d));
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     :
-                     : "s"(lds), "v"(voff), "s"(d));
+    return make_rsrc(base, bytes <= 0 ? 0u : (bytes > 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes));
 }
 
 // Until at most N of this wave's DMA requests are in flight and its LDS reads are done, then the
@@ -142,17 +121,16 @@ struct Gemm {
             const int r = (wave * TB::NI + i) * TB::RPI + rb;
             vb[i] = (uint32_t)r * (uint32_t)pb + (uint32_t)((cb ^ TB::swizzle(r)) << 4);
         }
-        const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
 
         // The requests of one step's tile, one at a time (q = 0 .. NDMA - 1).
         struct Tile {
             u32x4 da, db;
-            uint32_t lds;
+            const char* lds;
             int left;       // k left from this step on (chunks past K come from out of range, as zeros)
         };
         auto tile_at = [&](int t, int buf) __attribute__((always_inline)) {
             return Tile{desc(abase + t * astep, aend - t * astep), desc(bbase + t * bstep, bend - t * bstep),
-                        lds0 + buf * STAGE_BYTES, p.K - t * BK};
+                        smem + buf * STAGE_BYTES, p.K - t * BK};
         };
         auto request = [&](const Tile& x, int q) __attribute__((always_inline)) {
             if (q < TA::NI) {
@@ -161,8 +139,7 @@ struct Gemm {
                     const int r = (wave * TA::NI + q) * TA::RPI + ra;
                     if (x.left < BK) v = ((ca ^ TA::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
                 }
-                if (q == 0) dma_asm<true>(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
-                else dma_asm<false>(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
+                dma16(x.da, x.lds + (wave * TA::NI + q) * 1024, v, q == 0);
             } else {
                 const int i = q - TA::NI;
                 uint32_t v = vb[i];
@@ -170,8 +147,7 @@ struct Gemm {
                     const int r = (wave * TB::NI + i) * TB::RPI + rb;
                     if (x.left < BK) v = ((cb ^ TB::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
                 }
-                if (i == 0) dma_asm<true>(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
-                else dma_asm<false>(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
+                dma16(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v, i == 0);
             }
         };
 
