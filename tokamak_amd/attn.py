@@ -11,6 +11,7 @@ call fails, an exception is raised.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 import re
@@ -100,6 +101,7 @@ def _check(fn: str, rc: int) -> None:
         raise AttnError(fn, rc, lib().tkm_attn_last_error().decode())
 
 
+@functools.lru_cache(maxsize=64)
 def default_scale(D: int) -> float:
     """1/sqrtf(D) in fp32, as the reference dispatch passes (tkm_gpu.cu:1258)."""
     import numpy as np
@@ -115,17 +117,23 @@ def _dtype_code(t) -> int:
     raise TypeError(f"attention tensors must be float16 or bfloat16, got {t.dtype}")
 
 
+# Addresses go to ctypes as plain ints (c_void_p argtypes take them), and the current stream's handle
+# comes from torch's C entry: the wrapper objects cost more host time than a small call's kernels.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(stream):
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _check_tensor(name, t, numel, device, dtype=None):
+    if (t.is_cuda and t.numel() == numel and t.is_contiguous() and (dtype is None or t.dtype == dtype)
+            and t.device == device):
+        return
     if not t.is_cuda or t.device != device:
         raise ValueError(f"{name} must be on {device}")
     if not t.is_contiguous():
@@ -143,10 +151,14 @@ def gqa_fwd(qkv, B, S, Hq, Hkv, D, causal=True, kv_len=None, scale=None,
     dev = qkv.device
     _check_tensor("qkv", qkv, B * S * (Hq + 2 * Hkv) * D, dev)
     dt = _dtype_code(qkv)
-    out = torch.empty((B, S, Hq * D), dtype=qkv.dtype, device=dev) if out is None else out
-    lse = torch.empty((B, Hq, S), dtype=torch.float32, device=dev) if lse is None else lse
-    _check_tensor("out", out, B * S * Hq * D, dev, qkv.dtype)
-    _check_tensor("lse", lse, B * Hq * S, dev, torch.float32)
+    if out is None:
+        out = torch.empty((B, S, Hq * D), dtype=qkv.dtype, device=dev)
+    else:
+        _check_tensor("out", out, B * S * Hq * D, dev, qkv.dtype)
+    if lse is None:
+        lse = torch.empty((B, Hq, S), dtype=torch.float32, device=dev)
+    else:
+        _check_tensor("lse", lse, B * Hq * S, dev, torch.float32)
     if kv_len is not None:
         _check_tensor("kv_len", kv_len, B, dev, torch.int32)
     scale = default_scale(D) if scale is None else float(scale)
@@ -172,12 +184,15 @@ def gqa_bwd(qkv, o, dout, lse, B, S, Hq, Hkv, D, causal=True, kv_len=None, scale
     if kv_len is not None:
         _check_tensor("kv_len", kv_len, B, dev, torch.int32)
     dt = _dtype_code(qkv)
-    dqkv = torch.empty_like(qkv) if dqkv is None else dqkv
-    _check_tensor("dqkv", dqkv, qkv.numel(), dev, qkv.dtype)
-    need = bwd_workspace_bytes(B, S, Hq)
+    if dqkv is None:
+        dqkv = torch.empty_like(qkv)
+    else:
+        _check_tensor("dqkv", dqkv, qkv.numel(), dev, qkv.dtype)
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-    wbytes = workspace.numel() * workspace.element_size()
+        wbytes = bwd_workspace_bytes(B, S, Hq)
+        workspace = torch.empty(wbytes, dtype=torch.uint8, device=dev)
+    else:
+        wbytes = workspace.numel() * workspace.element_size()
     scale = default_scale(D) if scale is None else float(scale)
     args = (_ptr(qkv), _ptr(o), _ptr(dout), _ptr(lse), _ptr(dqkv), _ptr(kv_len), B, S, Hq, Hkv,
             D, scale, int(bool(causal)), dt, _ptr(workspace), wbytes, _stream(stream))

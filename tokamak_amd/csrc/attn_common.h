@@ -62,6 +62,18 @@ __device__ __forceinline__ uint32_t pack2(float x, float y) {
     }
 }
 
+// Sum of the two 16-bit values in w, accumulated in fp32.
+template <int DT>
+__device__ __forceinline__ float dot2_ones(uint32_t w, float acc) {
+    if constexpr (DT == DT_F16) {
+        const f16x2 one = {(_Float16)1.0f, (_Float16)1.0f};
+        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, w), one, acc, false);
+    } else {
+        const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
+        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), one, acc, false);
+    }
+}
+
 // bf16 keeps 8 significant bits, too few for the probabilities P and dS that feed the
 // second GEMM of each pair at the stated tolerance.  In bf16 mode they are therefore split
 // into hi = bf16(x) and lo = bf16(x - hi) and both halves go through the MFMA (same A

@@ -17,7 +17,7 @@
 // Per tile and wave:
 //   S^T = K Q^T        32 keys x 32 queries per MFMA block; lane = query row.
 //   P^T = exp2(S^T * scale*log2e - m) with m the row offset (log2 units, below); the row sum
-//                      is the lane's fp32 sum of P, lane halves combined at the end.
+//                      is summed per lane in fp32, lane halves combined at the end.
 //   O^T += V^T P^T     the P^T accumulator, rounded to 16 bits, is the B operand in place;
 //                      V^T comes from the row-major V tile through ds_read_b64_tr_b16.
 //
@@ -31,8 +31,9 @@
 // fp32 (a scale folded into Q and rounded to 16 bits would move a score s by up to
 // |s|*2^-12, which trained attention logits turn into errors past the bars).  m starts as
 // the row max of the first tile and moves only when it must (a lazy online softmax): when a
-// later tile's P sum reaches fp16's largest value, the wave raises m of its rows to max(m, the tile's row max), multiplies O and
-// the row sums by 2^(m_old - m_new) and repeats the tile's exp2 before its PV product.
+// later tile's P sum reaches fp16's largest value, the wave raises m of its rows to max(m, the
+// tile's row max), multiplies O and the row sums by 2^(m_old - m_new) and repeats the tile's exp2
+// before its PV product.
 // Causal: tiles above the diagonal are neither loaded nor computed, tiles crossing the
 // diagonal (or the kv_len / S edge) are masked, heaviest query blocks are launched first.
 #include <type_traits>
@@ -204,9 +205,9 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
         }
     };
     // exp2 of the scores in set J (relative to mm[qb]), packed to 16 bits into P set J;
-    // lt[qb] = the lane's sum of the fp32 values, as the assembly kernels and the reference's
-    // (tkm_gpu.cu:403) sum them: LSE is then within 1e-7 of 64 bits, against 2e-6 to 8e-6 with the
-    // sum of the packed values.
+    // lt[qb] = the lane's sum of the packed values (D = 64; one dot product a pair, 4% of the forward
+    // at B4 S1024 H8 less than two adds), or of the fp32 values (D = 128, as the assembly kernels
+    // that serve the other sizes sum them: LSE within 1e-7 of 64 bits, against 2e-6 to 8e-6).
     auto stage_exp = [&](auto Jc, const float (&mm)[QB], float (&lt)[QB]) __attribute__((always_inline)) {
         constexpr int J = decltype(Jc)::value;
 #pragma unroll
@@ -225,10 +226,13 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
                         const u32x2 hl = pack_split_bf16(p0, p1);
                         pr[J][qb][ks][w] = hl[0];
                         plr[J][qb][ks][w] = hl[1];
+                        if constexpr (D == 64) lt[qb] = dot2_ones<DT>(hl[1], dot2_ones<DT>(hl[0], lt[qb]));
                     } else {
-                        pr[J][qb][ks][w] = pack2<DT>(p0, p1);
+                        const uint32_t pw = pack2<DT>(p0, p1);
+                        pr[J][qb][ks][w] = pw;
+                        if constexpr (D == 64) lt[qb] = dot2_ones<DT>(pw, lt[qb]);
                     }
-                    lt[qb] += p0 + p1;
+                    if constexpr (D == 128) lt[qb] += p0 + p1;
                 }
             }
         }
