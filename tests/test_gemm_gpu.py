@@ -12,7 +12,8 @@ from attn_cases import log
 
 pytestmark = pytest.mark.gpu
 
-TILES = {"256x128": 0, "128x128": 1, "128x64": 2, "64x64": 3}
+TILES = {"auto": -1, "256x128": 0, "128x128": 1, "128x64": 2, "64x64": 3, "128x64 split": 4, "64x64 split": 5,
+         "64x64 split deep": 6}
 
 
 class Problem(ctypes.Structure):
@@ -53,6 +54,8 @@ def check(name, got, whole, ref, mag, K, bits):
 # rows, then the two layer sizes: single rows and chunks, tiles less and more one chunk, partial
 # k-steps, k shorter than the pipeline
 SHAPES = [(1, 8, 8), (65, 72, 40), (127, 136, 200), (128, 128, 64), (129, 264, 328), (300, 520, 136), (520, 64, 576)]
+# sizes whose own tile is a split one: 64x64, 64x64 of long sums, 128x64
+LONG = [(200, 64, 328), (70, 72, 2056), (4090, 384, 1032)]
 
 
 @pytest.mark.parametrize("tile", sorted(TILES))
@@ -63,7 +66,7 @@ def test_layer_products(gpu, tile, bf16, b_along_k, accumulate):
     import torch
     L = lib()
     dt = torch.bfloat16 if bf16 else torch.float16
-    for M, N, K in SHAPES:
+    for M, N, K in SHAPES + (LONG if tile == "auto" else []):
         log(f"[case] tile {tile} bf16={bf16} b_along_k={b_along_k} acc={accumulate} {M}x{N}x{K}")
         torch.manual_seed(M + N + K)
         A, _ = guarded((M, K), dt)

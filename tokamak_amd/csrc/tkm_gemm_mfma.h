@@ -20,7 +20,9 @@ typedef struct {
 } TkmGemmProblem;
 
 enum { TKM_GEMM_TILE_AUTO = -1, TKM_GEMM_TILE_256x128 = 0, TKM_GEMM_TILE_128x128 = 1, TKM_GEMM_TILE_128x64 = 2,
-       TKM_GEMM_TILE_64x64 = 3 };
+       TKM_GEMM_TILE_64x64 = 3,
+       /* two groups of waves on alternate k-steps; tkm_gemm_mfma_run only */
+       TKM_GEMM_TILE_128x64_SPLIT = 4, TKM_GEMM_TILE_64x64_SPLIT = 5, TKM_GEMM_TILE_64x64_SPLIT_DEEP = 6 };
 
 /* Whether the kernels take the shape: stored rows in multiples of 8 elements, offsets within a tile
  * in 32 bits.  weight_grad: the operands of tkm_gemm_mfma_group (any K), else of tkm_gemm_mfma_run. */
@@ -32,7 +34,7 @@ TKM_GEMM_MFMA_API int tkm_gemm_mfma_run(const TkmGemmProblem *p, int b_along_k, 
                                         void *stream);
 
 /* Weight gradients: A along m, B along n, fp32 C written.  `table` (device memory) holds n problems
- * with their first tiles; tile is not 128x64, tiles the total of tkm_gemm_mfma_tiles. */
+ * with their first tiles; tile is not 128x64 or a split one, tiles the total of tkm_gemm_mfma_tiles. */
 TKM_GEMM_MFMA_API long long tkm_gemm_mfma_tiles(const TkmGemmProblem *p, int tile);
 TKM_GEMM_MFMA_API int tkm_gemm_mfma_group(const TkmGemmProblem *table, int n, long long tiles, int bf16, int tile,
                                           void *stream);

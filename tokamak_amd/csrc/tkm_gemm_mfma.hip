@@ -18,15 +18,16 @@
 // place for every LDS read and request between the MFMAs (in one burst they hold the wave's issue: dW of
 // 4096 rows, 512 x 8192: 65 -> 46 us).
 // Measured in bf16 at rows 4096, against hipBLASLt's first choice in the same training step:
-//   forward  N 1536, K 512 : 12.8 us (17.5)     dX  N 512, K 1536 : 12.1 us (24.5)
+//   forward  N 1536, K 512 : 12.8 us (17.5)     dX  N 512, K 1536 : 11.5 us (24.5)
 //            N 512,  K 512 :  7.2 us (12.8)         N 512, K 512  :  6.9 us (10.4)
-//            N 2752, K 512 : 20.0 us (30)           N 512, K 2752 : 19.4 us (44)
-//            N 512, K 1376 : 12.0 us (21.3)         N 1376, K 512 : 11.4 us (31)
-//            N 8192, K 512 : 57 us (50)             N 512, K 8192 : 53 us (118)
+//            N 2752, K 512 : 20.0 us (30)           N 512, K 2752 : 18.9 us (44)
+//            N 512, K 1376 : 11.4 us (21.3)         N 1376, K 512 : 11.4 us (31)
+//            N 8192, K 512 : 57 us (50)             N 512, K 8192 : 44 us (118)
 // and 4096 x 4096 x 4096 at 1.04 PFLOP/s (256x128).  The 8-layer decoder's training step: 3676 -> 2910 us,
 // outputs equal bit for bit (the MFMA sums run over k in the same order).
 //
-// A workgroup is 4 waves in a 2 x 2 grid.  The product is formed transposed (the B operand's columns
+// A workgroup is 4 waves in a 2 x 2 grid, or two such groups that take the k-steps in turn and add their
+// sums through LDS (pick_tile).  The product is formed transposed (the B operand's columns
 // are the MFMA's rows), so a lane holds one row of C and 4 consecutive columns per register quad;
 // the tile leaves through LDS as fp32 rows, read back as whole 16-byte groups of columns.
 #include <hip/hip_runtime.h>
@@ -63,7 +64,7 @@ struct Operand {
     static __device__ __forceinline__ int swizzle(int r) { return swz<(COLS > 128 ? 128 : COLS)>(r); }
 };
 
-template <int DT, bool AKC, bool BKC, int BM, int BN, int STAGES, bool OUT32>
+template <int DT, bool AKC, bool BKC, int BM, int BN, int STAGES, bool OUT32, int GROUPS = 1>
 struct Gemm {
     using TA = Operand<AKC, BM>;
     using TB = Operand<BKC, BN>;
@@ -71,8 +72,14 @@ struct Gemm {
     static constexpr int NDMA = TA::NI + TB::NI;
     static constexpr int STAGE_BYTES = TA::BYTES + TB::BYTES;
     static constexpr int EPITCH = WN + 4;                       // fp32 staging row
-    static constexpr int EPI_BYTES = 4 * 32 * EPITCH * 4;
-    static constexpr int LDS_BYTES = STAGES * STAGE_BYTES > EPI_BYTES ? STAGES * STAGE_BYTES : EPI_BYTES;
+    static constexpr int EPI_BYTES = GROUPS * 4 * 32 * EPITCH * 4;
+    // the groups' exchange of partial sums: of each 4-wave group's MB blocks of rows, those the other stores
+    static constexpr int OWN = GROUPS == 2 && MB > 1 ? MB / 2 : MB;
+    static constexpr int XCH_BYTES = GROUPS == 2 ? 8 * OWN * NB * 4096 : 0;
+    static constexpr int TILE_BYTES = GROUPS * STAGES * STAGE_BYTES;
+    static constexpr int LDS_BYTES = TILE_BYTES > EPI_BYTES + XCH_BYTES ? TILE_BYTES : EPI_BYTES + XCH_BYTES;
+    static_assert(GROUPS == 1 || GROUPS == 2, "one or two wave groups");
+    static_assert(LDS_BYTES <= 160 * 1024, "LDS of one CU");
 
     // LDS reads of one MFMA operand (32 indices from idx0, 16 k of step ks): one of 16 bytes per lane
     // (KC) or two transposing ones of 8 (NC).
@@ -95,10 +102,11 @@ struct Gemm {
 
     static __device__ __forceinline__ void run(const TkmGemmProblem& p, int tm, int tn, int accumulate, char* smem) {
         const int tid = threadIdx.x, lane = tid & 63;
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3, grp = GROUPS == 1 ? 0 : wave8 >> 2;
         const int m0 = tm * BM, n0 = tn * BN;
         const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
-        const int nt = (p.K + BK - 1) / BK;
+        const int nt = ((p.K + BK - 1) / BK + GROUPS - 1) / GROUPS;   // steps of each group
+        char* const tiles = smem + grp * STAGES * STAGE_BYTES;
 
         // Bytes from one k-step's tile to the next, and from the tile's first byte to the tensor's end.
         const long long pa = 2ll * p.lda, pb = 2ll * p.ldb;
@@ -128,9 +136,10 @@ struct Gemm {
             const char* lds;
             int left;       // k left from this step on (chunks past K come from out of range, as zeros)
         };
-        auto tile_at = [&](int t, int buf) __attribute__((always_inline)) {
+        auto tile_at = [&](int step, int buf) __attribute__((always_inline)) {
+            const int t = step * GROUPS + grp;      // the groups take the k-steps in turn
             return Tile{desc(abase + t * astep, aend - t * astep), desc(bbase + t * bstep, bend - t * bstep),
-                        smem + buf * STAGE_BYTES, p.K - t * BK};
+                        tiles + buf * STAGE_BYTES, p.K - t * BK};
         };
         auto request = [&](const Tile& x, int q) __attribute__((always_inline)) {
             if (q < TA::NI) {
@@ -166,7 +175,7 @@ struct Gemm {
         constexpr int KSLOT = MB * NB, NSLOT = KST * KSLOT;                          // MFMAs per k-group, per step
         constexpr int MEET = KSLOT + (KSLOT + 1) / 2, REST = NSLOT - MEET;           // slot of the barrier, slots after
         auto read = [&](int stage, int ks, int q) __attribute__((always_inline)) {
-            const char* at = smem + stage * STAGE_BYTES;
+            const char* at = tiles + stage * STAGE_BYTES;
             if (q < MB * PA) piece<TA, AKC>(xa[ks][q / PA], at, wm + (q / PA) * 32, ks, q % PA, lane);
             else {
                 const int u = q - MB * PA;
@@ -213,12 +222,47 @@ struct Gemm {
         }
         wait_step<0>();
 
-        // acc[i][j]: lane row wm + i*32 + l32, columns wn + j*32 + g4*8 + hi*4 + 0..3 of register quad g4.
+        // Two groups: each hands the other the sums of the rows that the other stores (one block of rows:
+        // group 0 stores them all), lane by lane, past the staging rows.
+        const int own0 = GROUPS == 2 && MB > 1 ? grp * OWN : 0;
+        if constexpr (GROUPS == 2) {
+            float* xch = reinterpret_cast<float*>(smem + EPI_BYTES);
+            if (MB > 1 || grp == 1) {
+#pragma unroll
+                for (int i = 0; i < OWN; ++i)
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) {
+                        const f32x16 give = MB > 1 && grp == 1 ? acc[i][j] : acc[MB - OWN + i][j];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            *reinterpret_cast<f32x4*>(xch + ((((wave8 * OWN + i) * NB + j) * 4 + q) * 64 + lane) * 4) =
+                                f32x4{give[q * 4], give[q * 4 + 1], give[q * 4 + 2], give[q * 4 + 3]};
+                    }
+            }
+            __syncthreads();
+            if (MB == 1 && grp == 1) return;
+#pragma unroll
+            for (int i = 0; i < OWN; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    f32x16 keep = MB > 1 && grp == 1 ? acc[MB - OWN + i][j] : acc[i][j];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const f32x4 x = *reinterpret_cast<const f32x4*>(
+                            xch + (((((wave8 ^ 4) * OWN + i) * NB + j) * 4 + q) * 64 + lane) * 4);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) keep[q * 4 + e] += x[e];
+                    }
+                    acc[i][j] = keep;
+                }
+        }
+
+        // acc[i][j]: lane row wm + (own0 + i)*32 + l32, columns wn + j*32 + g4*8 + hi*4 + 0..3 of register quad g4.
         const int l32 = lane & 31, hi = lane >> 5;
-        float* st = reinterpret_cast<float*>(smem) + wave * 32 * EPITCH;
+        float* st = reinterpret_cast<float*>(smem) + wave8 * 32 * EPITCH;
         constexpr int VEC = OUT32 ? 4 : 8, CPW = WN / VEC, RPP = 64 / CPW;   // columns a lane stores, lanes per row
 #pragma unroll
-        for (int i = 0; i < MB; ++i) {
+        for (int i = 0; i < OWN; ++i) {
 #pragma unroll
             for (int j = 0; j < NB; ++j)
 #pragma unroll
@@ -229,7 +273,7 @@ struct Gemm {
 #pragma unroll
             for (int q = 0; q < 32 / RPP; ++q) {
                 const int r = q * RPP + lane / CPW, c = (lane % CPW) * VEC;
-                const int m = m0 + wm + i * 32 + r, n = n0 + wn + c;
+                const int m = m0 + wm + (own0 + i) * 32 + r, n = n0 + wn + c;
                 const f32x4 x = *reinterpret_cast<const f32x4*>(st + r * EPITCH + c);
                 if constexpr (OUT32) {
                     if (m < p.M && n < p.N) *reinterpret_cast<f32x4*>((float*)p.C + (size_t)m * p.ldc + n) = x;
@@ -263,10 +307,10 @@ __device__ __forceinline__ int xcd_tile(int w, int n) {
     return x * q + (x < r ? x : r) + (w >> 3);
 }
 
-template <int DT, bool AKC, bool BKC, int BM, int BN, int STAGES, bool OUT32>
-__global__ __launch_bounds__(256, BM * BN * STAGES >= 65536 ? 1 : 2)
+template <int DT, bool AKC, bool BKC, int BM, int BN, int STAGES, bool OUT32, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS, GROUPS == 2 || BM * BN * STAGES < 65536 ? 2 : 1)
 void k_gemm(TkmGemmProblem p, int accumulate) {
-    using G = Gemm<DT, AKC, BKC, BM, BN, STAGES, OUT32>;
+    using G = Gemm<DT, AKC, BKC, BM, BN, STAGES, OUT32, GROUPS>;
     __shared__ __attribute__((aligned(1024))) char smem[G::LDS_BYTES];
     const int tiles_n = (p.N + BN - 1) / BN;
     const int t = xcd_tile(blockIdx.x, gridDim.x);
@@ -296,10 +340,10 @@ long long tiles_of(const TkmGemmProblem& p, int bm, int bn) {
 
 int status() { return hipGetLastError() == hipSuccess ? 0 : -1; }
 
-template <int DT, bool BKC, int BM, int BN, int STAGES>
+template <int DT, bool BKC, int BM, int BN, int STAGES, int GROUPS = 1>
 int launch_t(const TkmGemmProblem& p, int accumulate, hipStream_t s) {
-    hipLaunchKernelGGL((k_gemm<DT, true, BKC, BM, BN, STAGES, false>), dim3((unsigned)tiles_of(p, BM, BN)), dim3(256), 0,
-                       s, p, accumulate);
+    hipLaunchKernelGGL((k_gemm<DT, true, BKC, BM, BN, STAGES, false, GROUPS>), dim3((unsigned)tiles_of(p, BM, BN)),
+                       dim3(256 * GROUPS), 0, s, p, accumulate);
     return status();
 }
 
@@ -310,10 +354,21 @@ int launch_t(const TkmGemmProblem& p, int accumulate, hipStream_t s) {
 //   N 512, K 2752 : 34, 30, 19, 25      128 tiles of 128x128 leave half the chip idle
 //   N 512, K 512  : 11, 8.4, 7.3, 7.6
 // and rows 200, N 512, K 2752 (where a step's latency counts): 32, 22, 18, 15.
+// With one workgroup a CU (the smaller tiles) a step takes about 900 cycles where its LDS reads need 384:
+// one wave a SIMD waits for each barrier.  Two wave groups that take the k-steps in turn fill those waits,
+// for one merge through LDS at the end (us, one group against two of 128x64, rows 4096, N 512):
+//   K 512: 6.9, 7.0   K 1376: 12.8, 11.4   K 1536: 12.9, 11.5   K 2752: 20.4, 18.9   K 8192: 54.0, 44.0
+// 64x64 (one group; two of 2 stages, so two workgroups fit a CU; two of 4 stages, one fits):
+//   rows 2048, N 512 : K 512 5.8 5.4 5.9   K 1376 10.4 8.7 9.1   K 2752 16.7 16.2 12.8   K 8192 43.2 38.1 29.9
+//   rows 200,  N 512 : K 512 5.5 5.1 5.5   K 1376 10.0 8.2 8.6   K 2752 16.4 11.5 12.0   K 8192 42.4 38.5 28.0
+//   rows 2048, N 128 : K 128 3.6 3.8 4.3   K 384   4.8 4.4 4.8   K 704   6.4  5.6  6.0
 int pick_tile(const TkmGemmProblem& p) {
     if (tiles_of(p, 256, 128) >= 512) return TKM_GEMM_TILE_256x128;
     if (tiles_of(p, 128, 128) >= 320) return TKM_GEMM_TILE_128x128;
-    return tiles_of(p, 128, 64) >= 192 ? TKM_GEMM_TILE_128x64 : TKM_GEMM_TILE_64x64;
+    const long long n = tiles_of(p, 128, 64);
+    if (n >= 192) return p.K >= 1024 && n <= 256 ? TKM_GEMM_TILE_128x64_SPLIT : TKM_GEMM_TILE_128x64;
+    if (p.K <= 256) return TKM_GEMM_TILE_64x64;
+    return p.K >= 2048 && tiles_of(p, 64, 64) <= 256 ? TKM_GEMM_TILE_64x64_SPLIT_DEEP : TKM_GEMM_TILE_64x64_SPLIT;
 }
 
 template <int DT, bool BKC>
@@ -322,6 +377,9 @@ int launch_tile(const TkmGemmProblem& p, int tile, int accumulate, hipStream_t s
         case TKM_GEMM_TILE_256x128: return launch_t<DT, BKC, 256, 128, 3>(p, accumulate, s);
         case TKM_GEMM_TILE_128x128: return launch_t<DT, BKC, 128, 128, 2>(p, accumulate, s);
         case TKM_GEMM_TILE_128x64: return launch_t<DT, BKC, 128, 64, 3>(p, accumulate, s);
+        case TKM_GEMM_TILE_128x64_SPLIT: return launch_t<DT, BKC, 128, 64, 3, 2>(p, accumulate, s);
+        case TKM_GEMM_TILE_64x64_SPLIT: return launch_t<DT, BKC, 64, 64, 2, 2>(p, accumulate, s);
+        case TKM_GEMM_TILE_64x64_SPLIT_DEEP: return launch_t<DT, BKC, 64, 64, 4, 2>(p, accumulate, s);
         default: return launch_t<DT, BKC, 64, 64, 4>(p, accumulate, s);
     }
 }
