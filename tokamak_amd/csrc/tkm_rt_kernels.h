@@ -39,6 +39,7 @@ int tkm_rt_fill_u32(void *dst, size_t bytes, uint32_t value, void *stream);
 /* Softmax + loss per row (loss_kind 0 CE, 1 focal with gamma, 2 MSE on the probabilities);
  * labels are uint8 or (label_i32) int32, one per row, or NULL (label 0).  Writes dlogits
  * (overwritten) unless is_eval, then loss_out / correct_out (added to them when acc_*). */
+__attribute__((visibility("default")))   /* for the tests of the kernel alone */
 int tkm_rt_softmax_loss(const void *logits, int dtype, const void *labels, int label_i32, void *dlogits,
                         float *row_loss, int *row_correct, int rows, int cols, int is_eval, int valid_rows,
                         int loss_kind, float gamma, float *loss_out, int *correct_out, int acc_loss,

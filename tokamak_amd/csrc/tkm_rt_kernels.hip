@@ -18,6 +18,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "attn_common.h"
 #include "tkm_rt_kernels.h"
 
 namespace {
@@ -142,16 +143,20 @@ __global__ __launch_bounds__(256) void k_softmax_loss(const uint16_t* __restrict
 // The same per-row softmax and loss for rows of a multiple of 8 columns, at most 8192: the
 // wave reads its row once into registers (16-byte loads, lane l holding columns
 // (64k + l)*8 .. +7 of chunk k) and runs max, sum and gradient from them, writing dlogits as
-// 16-byte stores.  Per element the arithmetic is the scalar kernel's; the sums run over each
-// lane's elements in column order, then over the wave.
-template <int NCH>
-__global__ __launch_bounds__(256) void k_softmax_loss_v(const uint16_t* __restrict__ logits, int dt,
+// 16-byte stores.  The sums run over each lane's elements in column order, then over the wave.
+// Bound by vector instructions (a wave's takes 4 cycles), so: each exponential is formed once and kept
+// in fp32; the quotient by the row's sum is a product with its reciprocal and one residual step,
+// which rounds as the division does; the label's term is formed in its own chunk only; and the
+// first-maximum test runs only in rows whose label holds the maximum.
+// 4096 x 8192 in bf16: 66 -> 46 us.
+template <int NCH, int DT>
+__global__ __launch_bounds__(256) void k_softmax_loss_v(const uint16_t* __restrict__ logits,
                                                         const void* __restrict__ labels, int label_i32,
                                                         uint16_t* __restrict__ dlogits, float* __restrict__ row_loss,
                                                         int* __restrict__ row_correct, int rows, int cols,
                                                         int is_eval, int valid_rows, int loss_kind, float gamma) {
     const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int r = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (r >= rows) return;
     const size_t base = (size_t)r * cols;
     const int nchunk = cols / 8;
@@ -164,47 +169,62 @@ __global__ __launch_bounds__(256) void k_softmax_loss_v(const uint16_t* __restri
     auto val = [&](const uint4& q, int j) __attribute__((always_inline)) {
         const int wi = j >> 1;
         const uint32_t w = wi == 0 ? q.x : (wi == 1 ? q.y : (wi == 2 ? q.z : q.w));
-        const uint16_t b = (uint16_t)((j & 1) ? (w >> 16) : (w & 0xffffu));
-        return dt == 1 ? __uint_as_float((uint32_t)b << 16) : __half2float(__ushort_as_half(b));
+        if (DT == 1) return __uint_as_float((j & 1) ? w & 0xffff0000u : w << 16);
+        return __half2float(__ushort_as_half((uint16_t)((j & 1) ? w >> 16 : w & 0xffffu)));
     };
     float mx = -1e30f;
-    int pred = 0x7fffffff;
-#pragma unroll
-    for (int k = 0; k < NCH; ++k) {
-        const int ch = k * 64 + lane;
-        if (ch < nchunk) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float v = val(x[k], j);
-                if (v > mx) { mx = v; pred = ch * 8 + j; }
-            }
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float om = __shfl_xor(mx, o, 64);
-        const int op = __shfl_xor(pred, o, 64);
-        if (om > mx || (om == mx && op < pred)) { mx = om; pred = op; }
-    }
-    if (pred == 0x7fffffff) pred = 0;
-    float sum = 0.f;
 #pragma unroll
     for (int k = 0; k < NCH; ++k)
         if (k * 64 + lane < nchunk) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) sum += expf(val(x[k], j) - mx);
+            for (int j = 0; j < 8; ++j) mx = fmaxf(mx, val(x[k], j));
         }
-    sum = wave_sum(sum);
+    mx = wave_max(mx);
     int lbl = 0;
     if (labels) lbl = label_i32 ? ((const int32_t*)labels)[r] : (int)((const uint8_t*)labels)[r];
     if (lbl < 0 || lbl >= cols) lbl = 0;
-    if (lane == 0) row_correct[r] = ((!is_eval || r < valid_rows) && pred == lbl) ? 1 : 0;
+    lbl = __builtin_amdgcn_readfirstlane(lbl);
+    const float vl = ld16(logits, base + lbl, DT);
+    // the label is the prediction when no column before it holds the maximum too (column 0 when no
+    // value exceeds the start of the maximum)
+    int correct = 0;
+    if (!(mx > -1e30f)) {
+        correct = lbl == 0;
+    } else if (vl == mx) {
+        int before = 0;
+#pragma unroll
+        for (int k = 0; k < NCH; ++k) {
+            const int ch = k * 64 + lane;
+            if (ch < nchunk) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) before |= ch * 8 + j < lbl && val(x[k], j) == mx;
+            }
+        }
+        correct = __ballot(before) == 0;
+    }
+    if (lane == 0) row_correct[r] = (!is_eval || r < valid_rows) ? correct : 0;
     if (is_eval) {
         if (lane == 0) row_loss[r] = 0.f;
         return;
     }
+    float e[NCH][8], sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k)
+        if (k * 64 + lane < nchunk) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                e[k][j] = expf(val(x[k], j) - mx);
+                sum += e[k][j];
+            }
+        }
+    sum = wave_sum(sum);
+    const float rsum = 1.0f / sum;
+    auto prob = [&](float ex) __attribute__((always_inline)) {
+        const float q = ex * rsum;
+        return fmaf(fmaf(-q, sum, ex), rsum, q);
+    };
     const float inv_rows = 1.0f / (float)rows;
-    float tp = expf(ld16(logits, base + lbl, dt) - mx) / sum;
+    float tp = expf(vl - mx) / sum;
     tp = fmaxf(tp, 1e-7f);
     const float fw = powf(1.0f - tp, gamma);
     const float fscale = loss_kind == 1 ? fw - gamma * tp * powf(1.0f - tp, gamma - 1.0f) * logf(tp) : 1.0f;
@@ -216,7 +236,7 @@ __global__ __launch_bounds__(256) void k_softmax_loss_v(const uint16_t* __restri
             if (ch < nchunk) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const float p = expf(val(x[k], j) - mx) / sum;
+                    const float p = prob(e[k][j]);
                     const float t = ch * 8 + j == lbl ? 1.0f : 0.0f;
                     brier += p * (p - t);
                     mse += (p - t) * (p - t) / (float)cols;
@@ -230,24 +250,28 @@ __global__ __launch_bounds__(256) void k_softmax_loss_v(const uint16_t* __restri
     for (int k = 0; k < NCH; ++k) {
         const int ch = k * 64 + lane;
         if (ch < nchunk) {
-            uint32_t w[4];
+            float g[8];
 #pragma unroll
-            for (int j2 = 0; j2 < 4; ++j2) {
-                uint16_t h2[2];
+            for (int j = 0; j < 8; ++j) g[j] = prob(e[k][j]);
+            if (loss_kind == 2) {
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const int j = 2 * j2 + e;
-                    const float p = expf(val(x[k], j) - mx) / sum;
-                    const float t = ch * 8 + j == lbl ? 1.0f : 0.0f;
-                    float g;
-                    if (loss_kind == 0) g = p - t;
-                    else if (loss_kind == 1) g = fscale * (p - t);
-                    else g = (2.0f / (float)cols) * p * ((p - t) - brier);
-                    h2[e] = to16(g * inv_rows, dt);
+                for (int j = 0; j < 8; ++j)
+                    g[j] = (2.0f / (float)cols) * g[j] * ((g[j] - (ch * 8 + j == lbl ? 1.0f : 0.0f)) - brier);
+            } else {
+                if (lbl >> 9 == k) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) g[j] -= ch * 8 + j == lbl ? 1.0f : 0.0f;
                 }
-                w[j2] = (uint32_t)h2[0] | ((uint32_t)h2[1] << 16);
+                if (loss_kind == 1) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) g[j] *= fscale;
+                }
             }
-            *(uint4*)(dlogits + base + (size_t)ch * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) g[j] *= inv_rows;
+            *(uint4*)(dlogits + base + (size_t)ch * 8) =
+                make_uint4(tkm::pack2<DT>(g[0], g[1]), tkm::pack2<DT>(g[2], g[3]), tkm::pack2<DT>(g[4], g[5]),
+                           tkm::pack2<DT>(g[6], g[7]));
         }
     }
     if (lane == 0) {
@@ -466,14 +490,12 @@ int tkm_rt_softmax_loss(const void* logits, int dtype, const void* labels, int l
     if (rows <= 0) return 0;
     const bool vec = cols % 8 == 0 && cols <= 8192 && ((uintptr_t)logits & 15u) == 0 &&
                      (is_eval || ((uintptr_t)dlogits & 15u) == 0);
-    if (vec && cols <= 2048)
-        hipLaunchKernelGGL(k_softmax_loss_v<4>, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)stream,
-                           (const uint16_t*)logits, dtype, labels, label_i32, (uint16_t*)dlogits, row_loss,
-                           row_correct, rows, cols, is_eval, valid_rows, loss_kind, gamma);
-    else if (vec)
-        hipLaunchKernelGGL(k_softmax_loss_v<16>, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)stream,
-                           (const uint16_t*)logits, dtype, labels, label_i32, (uint16_t*)dlogits, row_loss,
-                           row_correct, rows, cols, is_eval, valid_rows, loss_kind, gamma);
+    auto* kv = cols <= 2048 ? (dtype == 1 ? k_softmax_loss_v<4, 1> : k_softmax_loss_v<4, 0>)
+                            : (dtype == 1 ? k_softmax_loss_v<16, 1> : k_softmax_loss_v<16, 0>);
+    if (vec)
+        hipLaunchKernelGGL(kv, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)logits, labels,
+                           label_i32, (uint16_t*)dlogits, row_loss, row_correct, rows, cols, is_eval, valid_rows,
+                           loss_kind, gamma);
     else
         hipLaunchKernelGGL(k_softmax_loss, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)stream,
                            (const uint16_t*)logits, dtype, labels, label_i32, (uint16_t*)dlogits, row_loss,
