@@ -183,6 +183,17 @@ def test_plasma_config4_swiglu(gpu):
     run_chain(gpu, dict(C=1536, twin=True, left=["SiLU"], right=[], chain=[], acc=2), 4096, "f16", seed=41)
 
 
+@pytest.mark.parametrize("rows", (1, 33, 1027, 4099))
+@pytest.mark.parametrize("c", (dict(C=64, chain=["RMSNorm", "LayerScale"], acc=6),
+                               dict(C=256, chain=["Bias", "Add", "RMSNorm"], acc=7),
+                               dict(C=1376, twin=True, left=["SiLU"], right=[], chain=[], acc=1)),
+                         ids=lambda c: f"C{c['C']}")
+def test_plasma_row_bands(gpu, c, rows):
+    """Rows less and more than a pass of one block, and bands of several passes (narrow rows take 32 and
+    8 rows a pass, wide ones 4), with and without parameter partials."""
+    run_chain(gpu, c, rows, "bf16", seed=50 + rows, guard=True)
+
+
 def test_plasma_deterministic(gpu):
     import torch
     from tokamak_amd import plasma

@@ -675,7 +675,7 @@ static int plan_groups(TkmRuntime *rt) {
             tkm_prep_geometry(&d, &geo);
             G->gx = (unsigned)((geo.CH + 63) / 64);
             G->gy_fwd = (unsigned)((G->rows + 4 * TKM_PREP_FWD_RPW - 1) / (4 * TKM_PREP_FWD_RPW));
-            G->bands = (unsigned)tkm_bwd_bands(G->rows, (int)G->gx);
+            G->bands = (unsigned)tkm_bwd_bands(G->rows, (int)G->gx, 4, 1);
             G->gx_red = (unsigned)((geo.part_width + 63) / 64);
             G->part_bytes = TKM_ALIGN((size_t)G->bands * geo.part_width * sizeof(float));
             G->pw = geo.part_width;
@@ -693,7 +693,7 @@ static int plan_groups(TkmRuntime *rt) {
             G->gx = (unsigned)geo.XB;
             const int rpb = TKM_PLASMA_FWD_RPI * 4 * geo.RW;
             G->gy_fwd = (unsigned)((G->rows + rpb - 1) / rpb);
-            G->bands = (unsigned)tkm_bwd_bands(G->rows, geo.XB);
+            G->bands = (unsigned)tkm_bwd_bands(G->rows, geo.XB, 4 * geo.RW, geo.n_par > 0);
             G->gx_red = (unsigned)((geo.part_width + 63) / 64);
             G->part_bytes = geo.n_par ? TKM_ALIGN((size_t)G->bands * geo.part_width * sizeof(float)) : 0;
             G->pw = geo.part_width;

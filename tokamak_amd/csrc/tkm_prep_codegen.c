@@ -108,10 +108,11 @@ void tkm_prep_geometry(const tkm_prep_desc *d, tkm_prep_geom *g) {
     g->part_width = g->C + (d->has_qknorm ? g->QK : 0);
 }
 
-int tkm_bwd_bands(int rows, int xblocks) {
-    int bands = (TKM_BWD_TARGET_BLOCKS + xblocks - 1) / xblocks;
-    const int most = (rows + TKM_BWD_MIN_BAND - 1) / TKM_BWD_MIN_BAND;
-    if (bands > most) bands = most;
+int tkm_bwd_bands(int rows, int xblocks, int side, int partials) {
+    const int target = ((partials ? TKM_BWD_TARGET_BLOCKS : TKM_BWD_FREE_BLOCKS) + xblocks - 1) / xblocks;
+    int band = (rows + target - 1) / target;
+    band = band < side ? side : (band + side - 1) / side * side;
+    const int bands = (rows + band - 1) / band;
     return bands < 1 ? 1 : bands;
 }
 
