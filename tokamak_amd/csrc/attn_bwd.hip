@@ -158,7 +158,7 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
                 for (int i = 0; i < 32 / RPI; ++i) {
                     const int r = i * RPI + lane / CPR;
                     dma16(rv, &sV[wave][i * RPI * ROWB],
-                          (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4), i == 0);
+                          (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4));
                 }
             }
         }
@@ -179,8 +179,8 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
             for (int i = 0; i < NI; ++i) {
                 const int r0 = (wave * NI + i) * RPI, r = r0 + dma_r;
                 const uint32_t sw = (uint32_t)((dma_p ^ swz<D>(r)) << 4);
-                dma16(rq, &smem[grp][buf][0][r0 * ROWB], (uint32_t)r * ldb + sw, i == 0);
-                dma16(ro, &smem[grp][buf][1][r0 * ROWB], (uint32_t)r * ldob + sw, i == 0);
+                dma16(rq, &smem[grp][buf][0][r0 * ROWB], (uint32_t)r * ldb + sw);
+                dma16(ro, &smem[grp][buf][1][r0 * ROWB], (uint32_t)r * ldob + sw);
             }
             if (wave == 0) {
                 const size_t li = ((size_t)b * Hq + h) * S + qr0;
@@ -443,8 +443,8 @@ void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restri
         for (int i = 0; i < NI; ++i) {
             const int r0 = (wave * NI + i) * RPI, r = r0 + dma_r;
             const uint32_t voff = (uint32_t)r * ldb + (uint32_t)((dma_p ^ swz<D>(r)) << 4);
-            dma16(rk, &smem[grp][buf][0][r0 * ROWB], voff, i == 0);
-            dma16(rv, &smem[grp][buf][1][r0 * ROWB], voff, i == 0);
+            dma16(rk, &smem[grp][buf][0][r0 * ROWB], voff);
+            dma16(rv, &smem[grp][buf][1][r0 * ROWB], voff);
         }
     };
     const int fk = swz<D>(l32);

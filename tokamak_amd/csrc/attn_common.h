@@ -191,22 +191,19 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // wave-uniform).  In inline assembly, because the compiler follows the DMA builtin's LDS writes
 // conservatively: before the first transposed read (ld_lds_tr) after one it waits for every load in
 // flight, which ends the prefetch of the next tile in the middle of the current one.  The asm writes no
-// register; a tile's requests are awaited by wait_dma (or a counted wait) and a barrier before its
-// first read.  first: the descriptor may have just been written by a VALU lane read, which a buffer
-// access may follow only after 5 wait states; otherwise 1, between the write of m0 and its use.
-__device__ __forceinline__ void dma16(u32x4 r, const void* lds, uint32_t voffset, bool first = true) {
+// register but m0, which it names; a tile's requests are awaited by wait_dma (or a counted wait) and a
+// barrier before its first read.  The compiler's hazard pass does not look into it, so each block holds
+// the 5 wait states that a buffer access needs after a VALU lane read has written its descriptor: any word
+// of it may have come back from a spill just before, in front of the later requests of a tile too.
+__device__ __forceinline__ void dma16(u32x4 r, const void* lds, uint32_t voffset) {
     const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
-    if (first)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     : : "s"(at), "v"(voffset), "s"(r));
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     : : "s"(at), "v"(voffset), "s"(r));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 : : "s"(at), "v"(voffset), "s"(r) : "m0");
 }
 __device__ __forceinline__ void dma4(u32x4 r, const void* lds, uint32_t voffset) {
     const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds"
-                 : : "s"(at), "v"(voffset), "s"(r));
+                 : : "s"(at), "v"(voffset), "s"(r) : "m0");
 }
 // Wait until every memory operation of this wave, LDS DMA included, has completed.  The builtin, so
 // that the compiler knows its own loads done too and adds no wait for them inside the tile loop.

@@ -133,7 +133,7 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
         for (int i = 0; i < NI; ++i) {
             const int r0 = (gw * NI + i) * RPI, row = r0 + dma_r;
             dma16(r, &smem[grp][tensor][buf][r0 * ROWB],
-                  (uint32_t)row * ldb + (uint32_t)((dma_p ^ swz<D>(row)) << 4), i == 0);
+                  (uint32_t)row * ldb + (uint32_t)((dma_p ^ swz<D>(row)) << 4));
         }
     };
 

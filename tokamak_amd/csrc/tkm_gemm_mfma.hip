@@ -148,7 +148,7 @@ struct Gemm {
                     const int r = (wave * TA::NI + q) * TA::RPI + ra;
                     if (x.left < BK) v = ((ca ^ TA::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
                 }
-                dma16(x.da, x.lds + (wave * TA::NI + q) * 1024, v, q == 0);
+                dma16(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
             } else {
                 const int i = q - TA::NI;
                 uint32_t v = vb[i];
@@ -156,7 +156,7 @@ struct Gemm {
                     const int r = (wave * TB::NI + i) * TB::RPI + rb;
                     if (x.left < BK) v = ((cb ^ TB::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
                 }
-                dma16(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v, i == 0);
+                dma16(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
             }
         };
 
