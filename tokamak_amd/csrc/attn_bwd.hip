@@ -154,12 +154,13 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
             const auto rv = make_rsrc(bqkv + (size_t)kw0 * ld + (size_t)(Hq + Hkv + kvh) * D,
                                       rows_bytes(vrows, ldb, D * 2));
             if (grp == 0) {
+                uint32_t v[32 / RPI];
 #pragma unroll
                 for (int i = 0; i < 32 / RPI; ++i) {
                     const int r = i * RPI + lane / CPR;
-                    dma16(rv, &sV[wave][i * RPI * ROWB],
-                          (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4));
+                    v[i] = (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4);
                 }
+                dma16_rows(rv, lds_addr(sV) + (uint32_t)(wave * 32 * ROWB), v);
             }
         }
         const int qt_begin = causal ? kb0 / BM : 0;
@@ -168,24 +169,28 @@ void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __rest
         // group g takes iterations g, g + KSPLIT, ...; every group runs nit (barriers matched)
         const int nit = (iters + KSPLIT - 1) / KSPLIT;
 
-        const int dma_r = lane / CPR, dma_p = lane % CPR;
+        const uint32_t lds0 = lds_addr(smem) + (uint32_t)(grp * 4 * TILEB + wave * NI * 1024);
+        const uint32_t ld_lds = lds_addr(sLD) + (uint32_t)(grp * 1024);
         auto issue = [&](int it, int buf) __attribute__((always_inline)) {
             const int h = kvh * g + it / nq, qr0 = (qt_begin + it % nq) * BM;
             const uint32_t rows = (uint32_t)min(BM, S - qr0);
             const auto rq = make_rsrc(bqkv + (size_t)qr0 * ld + (size_t)h * D, rows_bytes(rows, ldb, D * 2));
             const auto ro = make_rsrc(dout + ((size_t)b * S + qr0) * ldo + (size_t)h * D,
                                       rows_bytes(rows, ldob, D * 2));
+            uint32_t vq[NI], vo[NI];
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
-                const int r0 = (wave * NI + i) * RPI, r = r0 + dma_r;
-                const uint32_t sw = (uint32_t)((dma_p ^ swz<D>(r)) << 4);
-                dma16(rq, &smem[grp][buf][0][r0 * ROWB], (uint32_t)r * ldb + sw);
-                dma16(ro, &smem[grp][buf][1][r0 * ROWB], (uint32_t)r * ldob + sw);
+                const int r = (wave * NI + i) * RPI + lane / CPR;
+                const uint32_t sw = (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4);
+                vq[i] = (uint32_t)r * ldb + sw;
+                vo[i] = (uint32_t)r * ldob + sw;
             }
+            dma16_rows(rq, lds0 + (uint32_t)(buf * 2 * TILEB), vq);
+            dma16_rows(ro, lds0 + (uint32_t)((buf * 2 + 1) * TILEB), vo);
             if (wave == 0) {
                 const size_t li = ((size_t)b * Hq + h) * S + qr0;
-                dma4(make_rsrc(lse + li, rows * 4), &sLD[grp][buf][0][0], (uint32_t)l32 * 4);
-                dma4(make_rsrc(delta + li, rows * 4), &sLD[grp][buf][1][0], (uint32_t)l32 * 4);
+                dma4(make_rsrc(lse + li, rows * 4), ld_lds + (uint32_t)(buf * 512), (uint32_t)l32 * 4);
+                dma4(make_rsrc(delta + li, rows * 4), ld_lds + (uint32_t)(buf * 512 + 256), (uint32_t)l32 * 4);
             }
         };
 
@@ -433,19 +438,20 @@ void fa_bwd_dq_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restri
     const int nit = (ntiles + KSPLIT - 1) / KSPLIT;
     const int tb = grp * nit, te = min(tb + nit, ntiles);
 
-    const int dma_r = lane / CPR, dma_p = lane % CPR;
+    const uint32_t lds0 = lds_addr(smem) + (uint32_t)(grp * 4 * TILEB + wave * NI * 1024);
+    uint32_t dma_v[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = (wave * NI + i) * RPI + lane / CPR;
+        dma_v[i] = (uint32_t)r * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(r)) << 4);
+    }
     auto issue = [&](int t, int buf) __attribute__((always_inline)) {
         const int k0 = t * BN;
         const uint32_t bytes = rows_bytes(min(BN, kv_end - k0), ldb, D * 2);
         const auto rk = make_rsrc(Kb + (size_t)k0 * ldb, bytes);
         const auto rv = make_rsrc(Vb + (size_t)k0 * ldb, bytes);
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int r0 = (wave * NI + i) * RPI, r = r0 + dma_r;
-            const uint32_t voff = (uint32_t)r * ldb + (uint32_t)((dma_p ^ swz<D>(r)) << 4);
-            dma16(rk, &smem[grp][buf][0][r0 * ROWB], voff);
-            dma16(rv, &smem[grp][buf][1][r0 * ROWB], voff);
-        }
+        dma16_rows(rk, lds0 + (uint32_t)(buf * 2 * TILEB), dma_v);
+        dma16_rows(rv, lds0 + (uint32_t)((buf * 2 + 1) * TILEB), dma_v);
     };
     const int fk = swz<D>(l32);
     const int trow = (lane & 15) >> 2;

@@ -187,23 +187,57 @@ __device__ __forceinline__ uint32_t rows_bytes(int rows, uint32_t pitch, uint32_
     return rows > 0 ? (uint32_t)(rows - 1) * pitch + width : 0u;
 }
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-// HBM -> LDS DMA: 16 (4) bytes per lane from rsrc + voffset to LDS at lds + 16 (4) * lane (lds is
+// LDS byte address of an object in shared memory, as one scalar (wave-uniform).  Taken once, of the whole
+// array: a pointer into it that depends on the wave stays a 64-bit generic one, with a null check before
+// each use, and a kernel's 16 or so of them spilled 26 to 45 scalar registers into the tile loop.
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)p);
+}
+// HBM -> LDS DMA: 16 (4) bytes per lane from rsrc + voffset to LDS at byte `at` + 16 (4) * lane (at is
 // wave-uniform).  In inline assembly, because the compiler follows the DMA builtin's LDS writes
 // conservatively: before the first transposed read (ld_lds_tr) after one it waits for every load in
 // flight, which ends the prefetch of the next tile in the middle of the current one.  The asm writes no
-// register but m0, which it names; a tile's requests are awaited by wait_dma (or a counted wait) and a
-// barrier before its first read.  The compiler's hazard pass does not look into it, so each block holds
-// the 5 wait states that a buffer access needs after a VALU lane read has written its descriptor: any word
-// of it may have come back from a spill just before, in front of the later requests of a tile too.
-__device__ __forceinline__ void dma16(u32x4 r, const void* lds, uint32_t voffset) {
-    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
+// register but m0 and scc, which it names; a tile's requests are awaited by wait_dma (or a counted wait)
+// and a barrier before its first read.  The compiler's hazard pass does not look into it, so each block
+// holds the 5 wait states that a buffer access needs after a VALU lane read has written its descriptor
+// (any word of it may have come back from a spill just before), and the one between a write of m0 and its use.
+__device__ __forceinline__ void dma16(u32x4 r, uint32_t at, uint32_t voffset) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  : : "s"(at), "v"(voffset), "s"(r) : "m0");
 }
-__device__ __forceinline__ void dma4(u32x4 r, const void* lds, uint32_t voffset) {
-    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
+__device__ __forceinline__ void dma4(u32x4 r, uint32_t at, uint32_t voffset) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds"
                  : : "s"(at), "v"(voffset), "s"(r) : "m0");
+}
+// For kernels that deal single requests out between their MFMAs, where 5 wait states each cost the wave's
+// issue (16 clocks a request: a 256x128 GEMM step 5%): dma_ready waits for what wrote two descriptors, once,
+// and the requests after it hold the state that m0 needs only.  The compiler moves scalars by scalar
+// instructions, but brings a spilled one back by a lane read, so this is for kernels that spill none
+// (tests/test_dma_asm.py asks the compiler).
+__device__ __forceinline__ void dma_ready(u32x4 a, u32x4 b) { asm volatile("s_nop 4" : : "s"(a), "s"(b)); }
+__device__ __forceinline__ void dma16_ready(u32x4 r, uint32_t at, uint32_t voffset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 : : "s"(at), "v"(voffset), "s"(r) : "m0");
+}
+// N requests of 16 bytes per lane from one descriptor, to 1024 consecutive bytes of LDS each.
+template <int N>
+__device__ __forceinline__ void dma16_rows(u32x4 r, uint32_t at, const uint32_t (&v)[N]) {
+    static_assert(N == 1 || N == 2 || N % 4 == 0, "requests in fours");
+    if constexpr (N == 1) dma16(r, at, v[0]);
+    if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+                     "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
+                     : : "s"(at), "v"(v[0]), "v"(v[1]), "s"(r) : "m0", "scc");
+    if constexpr (N >= 4) {
+#pragma unroll
+        for (int i = 0; i < N; i += 4)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
+                         "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
+                         "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %5, 0 offen lds\n\t"
+                         "s_add_u32 m0, m0, 1024\n\ts_nop 0\n\tbuffer_load_dwordx4 %4, %5, 0 offen lds"
+                         : : "s"(at + (uint32_t)i * 1024u), "v"(v[i]), "v"(v[i + 1]), "v"(v[i + 2]), "v"(v[i + 3]), "s"(r)
+                         : "m0", "scc");
+    }
 }
 // Wait until every memory operation of this wave, LDS DMA included, has completed.  The builtin, so
 // that the compiler knows its own loads done too and adds no wait for them inside the tile loop.

@@ -124,17 +124,18 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
 
     // DMA of one tile (tensor 0 = K, 1 = V) into buffer buf: wave w moves rows
     // [w*NI*RPI, (w+1)*NI*RPI) of the BN-row tile.
-    const int dma_r = lane / CPR, dma_p = lane % CPR;
+    const uint32_t lds0 = lds_addr(smem) + (uint32_t)(grp * 4 * TILEB + gw * NI * 1024);
+    uint32_t dma_v[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int row = (gw * NI + i) * RPI + lane / CPR;
+        dma_v[i] = (uint32_t)row * ldb + (uint32_t)(((lane % CPR) ^ swz<D>(row)) << 4);
+    }
     auto issue = [&](int t, int tensor, int buf) __attribute__((always_inline)) {
         const int k0 = t * BN;
         const auto r = make_rsrc((tensor ? Vb : Kb) + (size_t)k0 * ldb,
                                  rows_bytes(min(BN, kv_end - k0), ldb, D * 2));
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int r0 = (gw * NI + i) * RPI, row = r0 + dma_r;
-            dma16(r, &smem[grp][tensor][buf][r0 * ROWB],
-                  (uint32_t)row * ldb + (uint32_t)((dma_p ^ swz<D>(row)) << 4));
-        }
+        dma16_rows(r, lds0 + (uint32_t)((tensor * 2 + buf) * TILEB), dma_v);
     };
 
     // Per-lane LDS offsets.  K (A operand of S^T): row kb*32 + l32, chunk ks*2 + hi.
@@ -189,19 +190,20 @@ void fa_fwd_kernel(const uint16_t* __restrict__ qkv, uint16_t* __restrict__ out,
                     sr[J][kb][qb] = mfma32<DT>(a, qf[qb][ks], ks == 0 ? f32x16{} : sr[J][kb][qb]);
             }
     };
+    // Score register r of key block kb is key k0 + hi*4 + c of the lane's row, c a constant: hidden iff it is
+    // at or past the row's number of visible keys.
     auto stage_mask = [&](int t, auto Jc) __attribute__((always_inline)) {
         constexpr int J = decltype(Jc)::value;
         const int k0 = t * BN;
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
             const int q = q0 + qb * 32 + l32;
+            const int seen = (causal ? min(kvl, q + 1) : kvl) - k0 - hi * 4;
 #pragma unroll
             for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = k0 + kb * 32 + (r >> 2) * 8 + hi * 4 + (r & 3);
-                    if (key >= kvl || (causal && key > q)) sr[J][kb][qb][r] = -INFINITY;
-                }
+                for (int r = 0; r < 16; ++r)
+                    if (kb * 32 + (r >> 2) * 8 + (r & 3) >= seen) sr[J][kb][qb][r] = -INFINITY;
         }
     };
     // exp2 of the scores in set J (relative to mm[qb]), packed to 16 bits into P set J;

@@ -107,6 +107,7 @@ struct Gemm {
         const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
         const int nt = ((p.K + BK - 1) / BK + GROUPS - 1) / GROUPS;   // steps of each group
         char* const tiles = smem + grp * STAGES * STAGE_BYTES;
+        const uint32_t lds0 = lds_addr(smem) + (uint32_t)(grp * STAGES * STAGE_BYTES);
 
         // Bytes from one k-step's tile to the next, and from the tile's first byte to the tensor's end.
         const long long pa = 2ll * p.lda, pb = 2ll * p.ldb;
@@ -133,13 +134,13 @@ struct Gemm {
         // The requests of one step's tile, one at a time (q = 0 .. NDMA - 1).
         struct Tile {
             u32x4 da, db;
-            const char* lds;
+            uint32_t lds;
             int left;       // k left from this step on (chunks past K come from out of range, as zeros)
         };
         auto tile_at = [&](int step, int buf) __attribute__((always_inline)) {
             const int t = step * GROUPS + grp;      // the groups take the k-steps in turn
             return Tile{desc(abase + t * astep, aend - t * astep), desc(bbase + t * bstep, bend - t * bstep),
-                        tiles + buf * STAGE_BYTES, p.K - t * BK};
+                        lds0 + (uint32_t)(buf * STAGE_BYTES), p.K - t * BK};
         };
         auto request = [&](const Tile& x, int q) __attribute__((always_inline)) {
             if (q < TA::NI) {
@@ -148,7 +149,7 @@ struct Gemm {
                     const int r = (wave * TA::NI + q) * TA::RPI + ra;
                     if (x.left < BK) v = ((ca ^ TA::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
                 }
-                dma16(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
+                dma16_ready(x.da, x.lds + (wave * TA::NI + q) * 1024, v);
             } else {
                 const int i = q - TA::NI;
                 uint32_t v = vb[i];
@@ -156,7 +157,7 @@ struct Gemm {
                     const int r = (wave * TB::NI + i) * TB::RPI + rb;
                     if (x.left < BK) v = ((cb ^ TB::swizzle(r)) << 3) < x.left ? v : 0x80000000u;
                 }
-                dma16(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
+                dma16_ready(x.db, x.lds + TA::BYTES + (wave * TB::NI + i) * 1024, v);
             }
         };
 
@@ -186,6 +187,7 @@ struct Gemm {
 #pragma unroll
         for (int t = 0; t < STAGES; ++t) {
             const Tile tl = tile_at(t, t);
+            dma_ready(tl.da, tl.db);
 #pragma unroll
             for (int q = 0; q < NDMA; ++q) request(tl, q);
         }
@@ -198,6 +200,7 @@ struct Gemm {
         for (int t = 0; t < nt; ++t) {
             const int next = buf + 1 == STAGES ? 0 : buf + 1;
             const Tile tl = tile_at(t + STAGES, buf);
+            dma_ready(tl.da, tl.db);
 #pragma unroll
             for (int s = 0; s < NSLOT; ++s) {
                 const int ks = s / KSLOT, i = (s / NB) % MB, j = s % NB;
