@@ -24,9 +24,12 @@ enum { TKM_GEMM_TILE_AUTO = -1, TKM_GEMM_TILE_256x128 = 0, TKM_GEMM_TILE_128x128
        /* two groups of waves on alternate k-steps; tkm_gemm_mfma_run only */
        TKM_GEMM_TILE_128x64_SPLIT = 4, TKM_GEMM_TILE_64x64_SPLIT = 5, TKM_GEMM_TILE_64x64_SPLIT_DEEP = 6 };
 
-/* Whether the kernels take the shape: stored rows in multiples of 8 elements, offsets within a tile
- * in 32 bits.  weight_grad: the operands of tkm_gemm_mfma_group (any K), else of tkm_gemm_mfma_run. */
+/* Whether the kernels take the shape: stored rows in multiples of 8 elements, aligned pointers, offsets within
+ * a tile in 32 bits.  weight_grad: the operands of tkm_gemm_mfma_group (any K), else of tkm_gemm_mfma_run. */
 TKM_GEMM_MFMA_API int tkm_gemm_mfma_supported(const TkmGemmProblem *p, int weight_grad);
+
+/* Whether they also are the faster ones for it, against hipBLASLt: the runtime's choice. */
+TKM_GEMM_MFMA_API int tkm_gemm_mfma_preferred(const TkmGemmProblem *p, int weight_grad);
 
 /* A along k; B along k (b_along_k = 1) or along n.  16-bit C, written or (accumulate = 1) added to in
  * fp32.  tile: TKM_GEMM_TILE_*. */

@@ -405,8 +405,30 @@ extern "C" {
 int tkm_gemm_mfma_supported(const TkmGemmProblem* p, int weight_grad) {
     if (p->M < 1 || p->N < 1 || p->K < 1 || p->N % 8 || p->lda % 8 || p->ldb % 8 || p->ldc % 8) return 0;
     if (weight_grad ? p->M % 8 : p->K % 8) return 0;
+    if (((uintptr_t)p->A | (uintptr_t)p->B | (uintptr_t)p->C) & 15u) return 0;
     const long long lim = 1ll << 30;    // offsets of 256 stored rows, formed in 32 bits
     return 512ll * p->lda < lim && 512ll * p->ldb < lim && tiles_of(*p, 64, 64) < (1ll << 31);
+}
+
+// Measured in bf16 from a captured graph, operands out of cache, us of these kernels / of hipBLASLt:
+//   M x N x K
+//   4096 x 8192 x 512 :  63 / 46       4096 x 512 x 2752 : 22 / 26     4096 x 2752 x 512  : 25 / 29
+//   8192 x 2048 x 512 :  30 / 25       4096 x 1024 x 512 : 12 / 14     8192 x 768 x 2304  : 41 / 35
+//   2048 x 4096 x 4096:  77 / 70       2048 x 2048 x 2048: 29 / 26     8192 x 4096 x 4096 : 272 / 176
+// so large products, where its kernels' higher rate counts, are the library's from 6e9 multiply-adds on, of few
+// rows (bound by reading the other operand) later:
+//   128 x 4096 x 4096 :  24 / 39       128 x 4096 x 14336: 74 / 123    128 x 28672 x 4096 : 74 / 56
+// and long sums of few tiles, which it splits further:
+//   256 x 512 x 8192  :  35 / 15       256 x 1024 x 4096 : 20 / 12     512 x 1024 x 4096  : 21 / 16
+//   256 x 1024 x 2816 :  16 / 10       256 x 768 x 2304  : 11 / 9      512 x 1024 x 2816  : 16 / 15
+// Weight gradients by the size of the result:
+//   512 x 8192, rows 4096: 50 / 53     2048 x 2048: 45 / 52            3072 x 3072, rows 2048: 65 / 52
+int tkm_gemm_mfma_preferred(const TkmGemmProblem* p, int weight_grad) {
+    if (!tkm_gemm_mfma_supported(p, weight_grad)) return 0;
+    if (weight_grad) return (long long)p->M * p->N <= 1ll << 22;
+    const long long n = tiles_of(*p, 64, 64);
+    if ((p->K > 2048 && n <= 64) || (p->K > 3072 && p->M > 128 && n <= 128)) return 0;
+    return (double)p->M * p->N * p->K < (p->M <= 128 ? 10e9 : 6e9);
 }
 
 int tkm_gemm_mfma_run(const TkmGemmProblem* p, int b_along_k, int bf16, int tile, int accumulate, void* stream) {

@@ -9,7 +9,7 @@
  *
  * with this build's kernels: the generated qkv-prep and plasma epilogues (tkm_codegen_hip.c,
  * compiled by hipRTC for gfx950), the attention kernels (include/tkm_attn.h), the FC GEMMs
- * (tkm_gemm_mfma.hip, or hipBLASLt through tkm_gemm.hip for the shapes it does not take) and the
+ * (tkm_gemm_mfma.hip, or hipBLASLt through tkm_gemm.hip where that is faster or has to serve) and the
  * runtime's own kernels (tkm_rt_kernels.hip).  The step is captured once into a hipGraph and
  * replayed, as the reference does.  Host code is C; HIP is called through its C API.
  *
@@ -73,8 +73,8 @@ typedef struct {
     void *xhat;
     void *mask;
     float *lse;
-    /* an FC layer's three products: this build's kernels where they take the shape (own_*), else
-     * hipBLASLt (g_*) */
+    /* an FC layer's three products: this build's kernels where they are the faster ones (own_*,
+     * tkm_gemm_mfma_preferred), else hipBLASLt (g_*) */
     tkm_gemm *g_fwd, *g_dw, *g_dx;
     TkmGemmProblem p_fwd, p_dw, p_dx;
     int own_fwd, own_dw, own_dx;
@@ -586,7 +586,7 @@ static int plan_gemms(TkmRuntime *rt) {
         rt_tensor *t = &rt->tensors[st->t_w];
         uint8_t *x = rt->arena + g->nodes[n->in0].out_offset, *y = rt->arena + n->out_offset;
         st->p_fwd = (TkmGemmProblem){x, t->w16, y, rows, N, K, K, N, N, 0};
-        st->own_fwd = tkm_gemm_mfma_supported(&st->p_fwd, 0);
+        st->own_fwd = tkm_gemm_mfma_preferred(&st->p_fwd, 0);
         if (!st->own_fwd && tkm_gemm_create(&st->g_fwd, rt->lt, 0, 0, N, rows, K, N, K, N, ab, ab, 0.0f, TKM_GEMM_MAX_WS))
             goto fail;
         if (ws < tkm_gemm_workspace(st->g_fwd)) ws = tkm_gemm_workspace(st->g_fwd);
@@ -594,8 +594,8 @@ static int plan_gemms(TkmRuntime *rt) {
             uint8_t *dx = rt->grad_arena + g->nodes[n->in0].out_offset, *dy = rt->grad_arena + n->out_offset;
             st->p_dw = (TkmGemmProblem){x, dy, t->grad, K, N, rows, K, N, N, 0};
             st->p_dx = (TkmGemmProblem){dy, t->w16, dx, rows, K, N, N, N, K, 0};
-            st->own_dw = tkm_gemm_mfma_supported(&st->p_dw, 1);
-            st->own_dx = tkm_gemm_mfma_supported(&st->p_dx, 0);
+            st->own_dw = tkm_gemm_mfma_preferred(&st->p_dw, 1);
+            st->own_dx = tkm_gemm_mfma_preferred(&st->p_dx, 0);
             if (!st->own_dw && tkm_gemm_create(&st->g_dw, rt->lt, 0, 1, N, K, rows, N, K, N, ab, TKM_GEMM_F32, 0.0f,
                                                TKM_GEMM_MAX_WS))
                 goto fail;
@@ -617,7 +617,7 @@ static int plan_gemms(TkmRuntime *rt) {
     return 1;
 }
 
-/* The weight gradients of all GEMM nodes the kernels take, as one launch at the last of them in the
+/* The weight gradients of all GEMM nodes given to the kernels, as one launch at the last of them in the
  * backward walk.  Launched node by node (on `side`, next to the dX chain) each has too few tiles for
  * the chip, and its workgroups' LDS keeps the chain's GEMMs off their CUs: config 4's step took
  * 2978 us with six launches beside the chain, 2910 with one at its end.  Tile size by the total:
