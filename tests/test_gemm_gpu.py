@@ -12,8 +12,7 @@ from attn_cases import log
 
 pytestmark = pytest.mark.gpu
 
-TILES = {"auto": -1, "256x128": 0, "128x128": 1, "128x64": 2, "64x64": 3, "128x64 split": 4, "64x64 split": 5,
-         "64x64 split deep": 6}
+TILES = {"auto": -1, "256x128": 0, "128x128": 1, "128x64": 2, "64x64": 3, "128x64 split": 4, "64x64 split": 5}
 
 
 class Problem(ctypes.Structure):
@@ -54,8 +53,9 @@ def check(name, got, whole, ref, mag, K, bits):
 # rows, then the two layer sizes: single rows and chunks, tiles less and more one chunk, partial
 # k-steps, k shorter than the pipeline
 SHAPES = [(1, 8, 8), (65, 72, 40), (127, 136, 200), (128, 128, 64), (129, 264, 328), (300, 520, 136), (520, 64, 576)]
-# sizes whose own tile is a split one: 64x64, 64x64 of long sums, 128x64
-LONG = [(200, 64, 328), (70, 72, 2056), (4090, 384, 1032)]
+# sizes on either side of the lines of the tile's rule: 64x64 and its split form (K 768), the split 128x64, 128x128
+LONG = [(200, 64, 328), (200, 64, 760), (200, 64, 776), (70, 72, 2056), (4090, 384, 1032), (2560, 512, 1032),
+        (2552, 1656, 72)]
 
 
 @pytest.mark.parametrize("tile", sorted(TILES))

@@ -22,7 +22,7 @@ typedef struct {
 enum { TKM_GEMM_TILE_AUTO = -1, TKM_GEMM_TILE_256x128 = 0, TKM_GEMM_TILE_128x128 = 1, TKM_GEMM_TILE_128x64 = 2,
        TKM_GEMM_TILE_64x64 = 3,
        /* two groups of waves on alternate k-steps; tkm_gemm_mfma_run only */
-       TKM_GEMM_TILE_128x64_SPLIT = 4, TKM_GEMM_TILE_64x64_SPLIT = 5, TKM_GEMM_TILE_64x64_SPLIT_DEEP = 6 };
+       TKM_GEMM_TILE_128x64_SPLIT = 4, TKM_GEMM_TILE_64x64_SPLIT = 5 };
 
 /* Whether the kernels take the shape: stored rows in multiples of 8 elements, aligned pointers, offsets within
  * a tile in 32 bits.  weight_grad: the operands of tkm_gemm_mfma_group (any K), else of tkm_gemm_mfma_run. */

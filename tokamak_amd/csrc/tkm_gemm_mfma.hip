@@ -350,28 +350,34 @@ int launch_t(const TkmGemmProblem& p, int accumulate, hipStream_t s) {
     return status();
 }
 
-// Tile of one product, measured at rows 4096 in bf16 (us at 256x128, 128x128, 128x64, 64x64):
-//   N 8192, K 512 : 55, 66, 68, 97      four tiles of 256x128 a CU: the LDS reads of a larger wave
-//   N 2752, K 512 : 23, 20, 25, 35      tile (128x64) are the cheapest
-//   N 1536, K 512 : 13, 13, 15, 20      fewer tiles than that leave CUs idle in the last round
-//   N 512, K 2752 : 34, 30, 19, 25      128 tiles of 128x128 leave half the chip idle
-//   N 512, K 512  : 11, 8.4, 7.3, 7.6
-// and rows 200, N 512, K 2752 (where a step's latency counts): 32, 22, 18, 15.
+// Tile of one product, measured at rows 4096 in bf16, in cache (us at 256x128, 128x128, 128x64, 64x64):
+//   N 8192, K 512 : 57, 64, 66, 95      four tiles of 256x128 a CU: the LDS reads of a larger wave
+//   N 2752, K 512 : 22, 19, 22, 29      tile (128x64) are the cheapest
+//   N 1536, K 512 : 13, 12, 13, 17      fewer tiles than that leave CUs idle in the last round
+//   N 512, K 2752 : 33, 30, 18, 21      128 tiles of 128x128 leave half the chip idle
+//   N 512, K 512  : 11, 7.4, 6.5, 7.0
+// and rows 256, N 512, K 2752 (where a step's latency counts): 32, 21, 18, 15.
 // With one workgroup a CU (the smaller tiles) a step takes about 900 cycles where its LDS reads need 384:
 // one wave a SIMD waits for each barrier.  Two wave groups that take the k-steps in turn fill those waits,
-// for one merge through LDS at the end (us, one group against two of 128x64, rows 4096, N 512):
-//   K 512: 6.9, 7.0   K 1376: 12.8, 11.4   K 1536: 12.9, 11.5   K 2752: 20.4, 18.9   K 8192: 54.0, 44.0
-// 64x64 (one group; two of 2 stages, so two workgroups fit a CU; two of 4 stages, one fits):
-//   rows 2048, N 512 : K 512 5.8 5.4 5.9   K 1376 10.4 8.7 9.1   K 2752 16.7 16.2 12.8   K 8192 43.2 38.1 29.9
-//   rows 200,  N 512 : K 512 5.5 5.1 5.5   K 1376 10.0 8.2 8.6   K 2752 16.4 11.5 12.0   K 8192 42.4 38.5 28.0
-//   rows 2048, N 128 : K 128 3.6 3.8 4.3   K 384   4.8 4.4 4.8   K 704   6.4  5.6  6.0
+// for one merge through LDS at the end.  A layer's operands come from other CUs' writes and from memory, so
+// the lines are set by operands out of cache and by whole steps (us, one group / two; in cache):
+//   128x64, rows 4096, N 512:  K 1376 15.6 / 15.7 (11.8 / 12.1)   K 1536 15.2 / 15.6 (11.8 / 10.9)
+//                              K 2752 23.2 / 23.0 (19.7 / 18.2)   the decoder's step at 4096 rows 2770 / 2751
+//   64x64, rows 2048, N 512:   K 512 5.7 / 6.1 (5.5 / 5.5)        K 1376 10.8 / 11.2 (9.9 / 8.5)
+//                              K 1536 11.2 / 11.3 (10.4 / 8.7)    K 2752 16.1 / 16.2 (14.7 / 12.4)
+//          rows 256, N 512:    K 512 5.4 / 5.8 (5.2 / 5.2)        K 1376 9.6 / 8.7 (9.4 / 8.0)
+//                              K 1536 9.1 / 8.5 (9.2 / 7.9)       K 2752 14.0 / 12.0 (14.5 / 11.6)
+// A 64x64 form of two groups with two stages each, two workgroups of which fit a CU, led in cache up to K 1376
+// (rows 2048, K 1376: 8.0) and lost out of it, for want of loads in flight (13.0; K 2752: 22.1): the
+// decoder's step without it went from 1831 to 1788 us at 1024 rows and from 1541 to 1476 at 64.  The
+// lines of 256 tiles of 128x128 and of 160 of 128x64 are from the same runs (512 x 2752 x 512: 8.5 us at 64x64,
+// 6.5 at 128x64; 2048 x 2304 x 768: 19.9 at 128x64, 17.2 at 128x128).
 int pick_tile(const TkmGemmProblem& p) {
     if (tiles_of(p, 256, 128) >= 512) return TKM_GEMM_TILE_256x128;
-    if (tiles_of(p, 128, 128) >= 320) return TKM_GEMM_TILE_128x128;
+    if (tiles_of(p, 128, 128) >= 256) return TKM_GEMM_TILE_128x128;
     const long long n = tiles_of(p, 128, 64);
-    if (n >= 192) return p.K >= 1024 && n <= 256 ? TKM_GEMM_TILE_128x64_SPLIT : TKM_GEMM_TILE_128x64;
-    if (p.K <= 256) return TKM_GEMM_TILE_64x64;
-    return p.K >= 2048 && tiles_of(p, 64, 64) <= 256 ? TKM_GEMM_TILE_64x64_SPLIT_DEEP : TKM_GEMM_TILE_64x64_SPLIT;
+    if (n >= 160) return p.K >= 1024 && n <= 256 ? TKM_GEMM_TILE_128x64_SPLIT : TKM_GEMM_TILE_128x64;
+    return p.K < 768 || tiles_of(p, 64, 64) > 256 ? TKM_GEMM_TILE_64x64 : TKM_GEMM_TILE_64x64_SPLIT;
 }
 
 template <int DT, bool BKC>
@@ -381,8 +387,7 @@ int launch_tile(const TkmGemmProblem& p, int tile, int accumulate, hipStream_t s
         case TKM_GEMM_TILE_128x128: return launch_t<DT, BKC, 128, 128, 2>(p, accumulate, s);
         case TKM_GEMM_TILE_128x64: return launch_t<DT, BKC, 128, 64, 3>(p, accumulate, s);
         case TKM_GEMM_TILE_128x64_SPLIT: return launch_t<DT, BKC, 128, 64, 3, 2>(p, accumulate, s);
-        case TKM_GEMM_TILE_64x64_SPLIT: return launch_t<DT, BKC, 64, 64, 2, 2>(p, accumulate, s);
-        case TKM_GEMM_TILE_64x64_SPLIT_DEEP: return launch_t<DT, BKC, 64, 64, 4, 2>(p, accumulate, s);
+        case TKM_GEMM_TILE_64x64_SPLIT: return launch_t<DT, BKC, 64, 64, 4, 2>(p, accumulate, s);
         default: return launch_t<DT, BKC, 64, 64, 4>(p, accumulate, s);
     }
 }
