@@ -675,7 +675,8 @@ static int plan_groups(TkmRuntime *rt) {
             tkm_prep_geometry(&d, &geo);
             G->gx = (unsigned)((geo.CH + 63) / 64);
             G->gy_fwd = (unsigned)((G->rows + 4 * TKM_PREP_FWD_RPW - 1) / (4 * TKM_PREP_FWD_RPW));
-            G->bands = (unsigned)tkm_bwd_bands(G->rows, (int)G->gx, 4, 1);
+            G->band = tkm_bwd_band(G->rows, (int)G->gx, 4, 1);
+            G->bands = (unsigned)tkm_bwd_bands(G->rows, G->band);
             G->gx_red = (unsigned)((geo.part_width + 63) / 64);
             G->part_bytes = TKM_ALIGN((size_t)G->bands * geo.part_width * sizeof(float));
             G->pw = geo.part_width;
@@ -693,7 +694,8 @@ static int plan_groups(TkmRuntime *rt) {
             G->gx = (unsigned)geo.XB;
             const int rpb = TKM_PLASMA_FWD_RPI * 4 * geo.RW;
             G->gy_fwd = (unsigned)((G->rows + rpb - 1) / rpb);
-            G->bands = (unsigned)tkm_bwd_bands(G->rows, geo.XB, 4 * geo.RW, geo.n_par > 0);
+            G->band = tkm_bwd_band(G->rows, geo.XB, 4 * geo.RW, geo.n_par > 0);
+            G->bands = (unsigned)tkm_bwd_bands(G->rows, G->band);
             G->gx_red = (unsigned)((geo.part_width + 63) / 64);
             G->part_bytes = geo.n_par ? TKM_ALIGN((size_t)G->bands * geo.part_width * sizeof(float)) : 0;
             G->pw = geo.part_width;
@@ -704,7 +706,6 @@ static int plan_groups(TkmRuntime *rt) {
                 G->par_node[p] = geo.par[p].node;
             }
         }
-        G->band = (G->rows + G->bands - 1) / G->bands;
         if (G->n_par > 0) {
             snprintf(name, sizeof name, "tkm_plasma_bwd_g%d_reduce", gid);
             if (tkm_rtc_function(rt->module, name, &G->reduce)) return 0;

@@ -10,7 +10,7 @@
  *     its sums are DPP adds inside the lane row; every lane runs the reductions (lanes past
  *     the row end hold zeros), only loads and stores are predicated;
  *   - forward: 4 rows per lane slot, loads first;
- *   - backward: rows in bands of whole passes of the block (tkm_bwd_bands);
+ *   - backward: rows in bands of whole passes of the block (tkm_bwd_band);
  *     parameter-gradient sums stay in registers over the band, the block's lane slots combine
  *     through LDS in a fixed order into one partial row per band, and a reduce kernel (16
  *     waves per column group) adds the bands in order (no atomics).

@@ -121,7 +121,8 @@ int tkm_plasma_fwd(const tkm_plasma *p, void *const *args, int rows, void *strea
 
 size_t tkm_plasma_bwd_workspace_bytes(const tkm_plasma *p, int rows) {
     if (!p || rows < 0 || p->geom.n_par == 0) return 0;
-    size_t b = (size_t)tkm_bwd_bands(rows, p->geom.XB, 4 * p->geom.RW, 1) * (size_t)p->geom.part_width * sizeof(float);
+    const int bands = tkm_bwd_bands(rows, tkm_bwd_band(rows, p->geom.XB, 4 * p->geom.RW, 1));
+    size_t b = (size_t)bands * (size_t)p->geom.part_width * sizeof(float);
     return (b + 255) & ~(size_t)255;
 }
 
@@ -143,8 +144,8 @@ int tkm_plasma_bwd(const tkm_plasma *p, void *const *args, int rows, int acc_fla
     if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15u)))
         return tkm_set_error(TKM_ATTN_EWORKSPACE, "tkm_plasma_bwd: a 16-byte aligned workspace of %zu bytes is needed",
                              need);
-    const int bands = tkm_bwd_bands(rows, g->XB, 4 * g->RW, g->n_par > 0);
-    int band = (rows + bands - 1) / bands;
+    int band = tkm_bwd_band(rows, g->XB, 4 * g->RW, g->n_par > 0);
+    const int bands = tkm_bwd_bands(rows, band);
     float *part = (float *)workspace;
     if (rows > 0 || g->n_par > 0) {
         void *kargs[TKM_PLASMA_MAX_ARGS + 4];

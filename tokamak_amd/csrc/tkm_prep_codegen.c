@@ -12,8 +12,8 @@
  *     are DPP reductions inside a lane row (tkm_sum_lanes8/16), no LDS;
  *   - bias, gamma and the RoPE frequencies of the chunk are loaded once per lane;
  *   - forward: 4 rows per wave, all loads issued before the arithmetic;
- *   - backward: the d(bias) / d(gamma) sums stay in registers over the band (about 2048
- *     blocks in all, at least 16 rows per band), then the 4 waves combine through LDS in a
+ *   - backward: the d(bias) / d(gamma) sums stay in registers over the band (whole passes of
+ *     the 4 waves: tkm_bwd_band), then the 4 waves combine through LDS in a
  *     fixed order into one partial per band; a second kernel (16 waves per column group)
  *     adds the partials in band order.  No atomics: bitwise reproducible.
  * The RoPE inverse frequencies are computed here, on the host, in fp32 with the reference's
@@ -108,13 +108,13 @@ void tkm_prep_geometry(const tkm_prep_desc *d, tkm_prep_geom *g) {
     g->part_width = g->C + (d->has_qknorm ? g->QK : 0);
 }
 
-int tkm_bwd_bands(int rows, int xblocks, int side, int partials) {
+int tkm_bwd_band(int rows, int xblocks, int side, int partials) {
     const int target = ((partials ? TKM_BWD_TARGET_BLOCKS : TKM_BWD_FREE_BLOCKS) + xblocks - 1) / xblocks;
-    int band = (rows + target - 1) / target;
-    band = band < side ? side : (band + side - 1) / side * side;
-    const int bands = (rows + band - 1) / band;
-    return bands < 1 ? 1 : bands;
+    const int band = (rows + target - 1) / target;
+    return band < side ? side : (band + side - 1) / side * side;
 }
+
+int tkm_bwd_bands(int rows, int band) { return rows < 1 ? 1 : (rows + band - 1) / band; }
 
 static const char *kind(const tkm_prep_desc *d) { return d->dtype == TKM_ATTN_BF16 ? "bf16" : "f16"; }
 

@@ -31,16 +31,18 @@ typedef struct {
 
 TKM_HIDDEN int tkm_prep_check_desc(const tkm_prep_desc *d);
 TKM_HIDDEN void tkm_prep_geometry(const tkm_prep_desc *d, tkm_prep_geom *g);
-/* Bands (block rows of a backward) for `rows` rows and `xblocks` blocks across a row; `side` is the
+/* Rows of a band (a block row of a backward) for `rows` rows and `xblocks` blocks across a row; `side` is the
  * rows that a block takes side by side, `partials` whether each band leaves a row of parameter
- * partials.  A band is a multiple of `side`, so that no part of a block idles in its last pass, and
- * no more than one pass where the target blocks allow it: the rows a wave walks one after the other
- * cost more than the larger partials' reduction (4096 x 512: 446 us for 49 backwards against 528 at
- * four passes).  Before, 4096 rows of three blocks gave bands of 6 rows, two passes of which half of
- * the second was idle, and rows of 256 channels filled half of each block.
+ * partials.  A band is a multiple of `side`, so that no part of a block idles in its last pass (but the last
+ * band's, which may be short), and no more than one pass where the target blocks allow it: the rows a wave
+ * walks one after the other cost more than the larger partials' reduction (4096 x 512: 446 us for 49
+ * backwards against 528 at four passes).  Before, 4096 rows of three blocks gave bands of 6 rows, two passes
+ * of which half of the second was idle, and rows of 256 channels filled half of each block.
  * 4096 rows: qkv-prep of 1536 channels 13.3 -> 12.4 us and its reduction 5.8 -> 4.0, gated pair of 1376
- * 13.5 -> 12.0; the epilogues of one decoder layer 85.7 -> 80.6 us, the 8-layer step 2042 -> 2015. */
-TKM_HIDDEN int tkm_bwd_bands(int rows, int xblocks, int side, int partials);
+ * 13.5 -> 12.0; the epilogues of one decoder layer 85.7 -> 80.6 us. */
+TKM_HIDDEN int tkm_bwd_band(int rows, int xblocks, int side, int partials);
+/* Bands of `rows` rows, at least one. */
+TKM_HIDDEN int tkm_bwd_bands(int rows, int band);
 TKM_HIDDEN float tkm_rope_inv_freq(const tkm_prep_desc *d, int i);
 
 /* Checks that the current device is gfx950, compiles src with hipRTC and loads it; *module

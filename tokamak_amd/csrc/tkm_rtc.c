@@ -215,7 +215,8 @@ int tkm_prep_fwd(const tkm_prep *p, const void *in, void *out, const float *bias
 
 size_t tkm_prep_bwd_workspace_bytes(const tkm_prep *p, int rows) {
     if (!p || rows < 0) return 0;
-    size_t b = (size_t)tkm_bwd_bands(rows, (p->geom.CH + 63) / 64, 4, 1) * (size_t)p->geom.part_width * sizeof(float);
+    const int bands = tkm_bwd_bands(rows, tkm_bwd_band(rows, (p->geom.CH + 63) / 64, 4, 1));
+    size_t b = (size_t)bands * (size_t)p->geom.part_width * sizeof(float);
     return (b + 255) & ~(size_t)255;
 }
 
@@ -241,8 +242,8 @@ int tkm_prep_bwd(const tkm_prep *p, const void *dout, void *din, const void *sav
     if (!workspace || workspace_bytes < need)
         return tkm_set_error(TKM_ATTN_EWORKSPACE, "tkm_prep_bwd: workspace of %zu bytes needed, %zu given", need,
                              workspace ? workspace_bytes : (size_t)0);
-    int bands = tkm_bwd_bands(rows, (p->geom.CH + 63) / 64, 4, 1);
-    int band = (rows + bands - 1) / bands;
+    int band = tkm_bwd_band(rows, (p->geom.CH + 63) / 64, 4, 1);
+    int bands = tkm_bwd_bands(rows, band);
     float *part = (float *)workspace;
     void *a1[] = {(void *)&dout, (void *)&din, (void *)&save_xhat, (void *)&save_istd, (void *)&gamma,
                   (void *)&part, (void *)&rows, (void *)&band, (void *)&accumulate};
