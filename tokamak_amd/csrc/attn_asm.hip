@@ -14,10 +14,11 @@
 // recorded into the graph.  Kernels are launched with hipModuleLaunchKernel on the caller's
 // stream; a launch allocates nothing.
 //
-// They serve D = 128, fp16 and bf16, whose offsets fit the
-// kernels' 32-bit buffer offsets; every other configuration goes to the HIP kernels
-// (attn_fwd.hip, attn_bwd.hip).  On a gfx950 device a
-// failed load is an error (kAsmLoadError), never a silent switch to the HIP kernels.
+// They serve D = 128, fp16 and bf16, where the rules of attn_launch.h (pick_rows_form, pick_keys_form) give
+// them the call -- grids that their 256-row items fill, and the smallest calls -- and the offsets fit
+// their 32-bit buffer offsets; every other configuration goes to the HIP kernels (attn_fwd.hip,
+// attn_bwd.hip).  On a gfx950 device a failed load is an error (kAsmLoadError), never a silent
+// switch to the HIP kernels.
 #include <mutex>
 #include <stdio.h>
 #include <stdint.h>

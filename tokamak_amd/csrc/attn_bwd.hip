@@ -97,6 +97,11 @@ __global__ __launch_bounds__(256) void fa_bwd_delta_kernel(const uint16_t* __res
 // before group 0 writes them.  Blocks have 32 NW keys; with NW = 2 and causal they are numbered so that
 // the workgroups the dispatcher puts on one CU (blocks i and i + grid/2) pair a heavy (early) key
 // block with a light one.  attn_launch.h (pick_keys_form) has the choice and its measurements.
+// The tiles' DMA stays in flight through the tile before (attn_common.h), which against the compiler's
+// builtin gives 1x4 at D 64 up to 11% (B2 S4096 Hq32 Hkv8 causal 534 -> 478 us; B2 S1101 H32 not causal
+// 89 -> 79), and costs it 2 to 5% in fp16, not causal, where the grid is one even round of two workgroups a
+// CU (B2 S4096 Hq32 Hkv8: 626 -> 656), whose phases the builtin's early wait keeps apart; waiting early in
+// that case only did not bring it back (653 to 659).
 template <int D, int DT, int KSPLIT, int NW>
 __global__ __launch_bounds__(64 * NW * KSPLIT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fa_bwd_dkdv_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ dout,

@@ -71,9 +71,14 @@ enum HipForm { kForm1x4, kForm2x4, kForm2x2, kForm4x2, kForm8x1, kForm4x1, kForm
 //                  q 256, S 1024: 27.9; 27.3 24.9 30.9 45.7        36.0; 39.5 32.7 37.9 51.9
 //                  q 512, S 2048: 51.8; 54.4 52.8 75.2             68.6; 80.2 70.4 96.0
 //                  q 64,  S 512 : 16.9; 15.6 15.2 12.5 11.7        22.6; 21.8 20.0 15.9 13.3
-// The smallest D 128 calls (forward q <= 64, dQ q <= 48, S < 768) stay on the assembly kernels, the path
-// this library states for head dim 128 there (tests/test_attn_gpu.py, tests/test_graph_gpu.py),
-// although the split forms measured faster.
+// The smallest D 128 calls (S < 768, forward q <= 64, dQ q <= 48) stay on the assembly kernels although the
+// split forms are the faster ones there: that is the path that tests/test_attn_gpu.py,
+// tests/test_graph_gpu.py and tests/test_trained_attention_gpu.py hold the library to (q 12 and 32 in the
+// first two, forward q 64 at most in the third).  The two bounds come from those shapes and not from a
+// measurement; a call between them (q 64, S 512) runs its forward on the assembly and its dQ split, which
+// costs the forward 16.8 us for 11.7.
+// The figures above are of before the tile loop's scalar work fell; the forward's split forms and 1x4 have
+// since gained 2 to 6% (D 64 q 256, S 1024: 2x2 11.6, bf16 13.6; D 128 q 256, S 1024: 2x4 21.9).
 inline HipForm pick_rows_form(int D, bool dq, long long q, int S, bool causal, int n) {
     if (D == 128) {
         if ((q <= (dq ? 48 : 64) && S < 768) || q > n) return kFormAsm;
@@ -96,7 +101,8 @@ inline HipForm pick_rows_form(int D, bool dq, long long q, int S, bool causal, i
 //   D 128 (assembly; 4x1): k 12, S 700, g 8: 102; 79.3       k 32, S 512, g 2: 23.9; 21.0
 //         k 64, S 1024, g 4: 76.9; 61.6                      k 256, S 512, g 1: 18.0; 46.0
 //         k 128, S 2048, g 4: 148; 128, not causal 160; 241  k 144, S 1531, g 4: 113; 126
-// and the smallest calls stay on the assembly kernel as above.
+// and the smallest calls (k <= 24, lists under 2048 rows) stay on the assembly kernel for the reason above: the
+// bounds are those tests' shapes (k 6 and 16), and k 32, S 512, g 2 shows what they cost.
 inline HipForm pick_keys_form(int D, long long k, int S, int g, bool causal, int n) {
     const long long list = (long long)g * S;   // query rows a key block meets (not causal)
     if (D == 128) {

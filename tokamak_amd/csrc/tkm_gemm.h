@@ -1,4 +1,4 @@
-/* The runtime's GEMMs (tkm_gemm.hip, hipBLASLt): column-major C = op(A) . op(B) with
+/* The runtime's library GEMMs (tkm_gemm.hip, hipBLASLt): column-major C = op(A) . op(B) with
  * alpha = 1 and a fixed beta, the algorithm chosen at creation.  Returns 0 or -1 with
  * tkm_gemm_last_error(). */
 #ifndef TKM_GEMM_H

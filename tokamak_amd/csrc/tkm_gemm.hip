@@ -1,4 +1,5 @@
-// tkm_gemm.hip -- the runtime's FC GEMMs through hipBLASLt (host code; the C runtime calls the
+// tkm_gemm.hip -- FC GEMMs through hipBLASLt, for the products that the runtime's own kernels do not take or
+// are slower at (tkm_gemm_mfma_preferred in tkm_gemm_mfma.hip; host code, the C runtime calls the
 // extern "C" functions of tkm_gemm.h).  They replace the reference's cublasGemmEx calls
 // (src/tkm_gpu.cu:1207-1217 forward, 1330-1345 backward), with the same column-major
 // operands: a weight W is stored as the column-major N_out x K matrix (ld N_out), i.e. the

@@ -17,14 +17,15 @@
 // reads.  Hence several tile sizes (pick_tile), STAGES k-steps of LDS with STAGES - 1 in flight, a fixed
 // place for every LDS read and request between the MFMAs (in one burst they hold the wave's issue: dW of
 // 4096 rows, 512 x 8192: 65 -> 46 us).
-// Measured in bf16 at rows 4096, against hipBLASLt's first choice in the same training step:
-//   forward  N 1536, K 512 : 12.8 us (17.5)     dX  N 512, K 1536 : 11.5 us (24.5)
-//            N 512,  K 512 :  7.2 us (12.8)         N 512, K 512  :  6.9 us (10.4)
-//            N 2752, K 512 : 20.0 us (30)           N 512, K 2752 : 18.9 us (44)
-//            N 512, K 1376 : 11.4 us (21.3)         N 1376, K 512 : 11.4 us (31)
-//            N 8192, K 512 : 57 us (50)             N 512, K 8192 : 44 us (118)
-// and 4096 x 4096 x 4096 at 1.04 PFLOP/s (256x128).  The 8-layer decoder's training step: 3676 -> 2910 us,
-// outputs equal bit for bit (the MFMA sums run over k in the same order).
+// Measured in bf16 at rows 4096 from a captured graph, operands out of cache, against hipBLASLt's first choice:
+//   forward  N 1536, K 512 : 14.9 us (17.2)     dX  N 512, K 1536 : 15.1 us (17.4)
+//            N 512,  K 512 :  7.4 us (11.6)         N 512, K 512  :  7.3 us (11.0)
+//            N 2752, K 512 : 24.8 us (28.9)         N 512, K 2752 : 22.3 us (26.2)
+//            N 512, K 1376 : 15.3 us (19.9)         N 1376, K 512 : 13.9 us (19.6)
+// and 8192 x 4096 x 4096 in 272 us, 1.01 PFLOP/s (256x128), where the library takes 176: tkm_gemm_mfma_preferred
+// has the line between the two.  The 8-layer decoder's training step, one runtime: 3690 us with hipBLASLt,
+// 2750 with these kernels and the attention kernels' wave groups.  A tile of one wave group sums over k in order
+// (its outputs equalled the library's bit for bit); two groups each sum every other k-step.
 //
 // A workgroup is 4 waves in a 2 x 2 grid, or two such groups that take the k-steps in turn and add their
 // sums through LDS (pick_tile).  The product is formed transposed (the B operand's columns
@@ -54,13 +55,13 @@ __device__ __forceinline__ void wait_step() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
-// LDS layout of one operand tile.  KC: IDX rows of BK values; NC: BK rows of IDX values (IDX <= 128).
+// LDS layout of one operand tile.  KC: IDX rows of BK values; NC: BK rows of IDX values.
 template <bool KC, int IDX>
 struct Operand {
     static constexpr int ROWS = KC ? IDX : BK, COLS = KC ? BK : IDX;
     static constexpr int ROWB = COLS * 2, CPR = COLS / 8, BYTES = ROWS * ROWB;
     static constexpr int RPI = 64 / CPR, NI = ROWS / RPI / 4;   // rows per DMA request, requests per wave
-    static_assert(COLS == 64 || COLS == 128 || COLS == 256, "tile rows of 128 or 256 bytes");
+    static_assert(COLS == 64 || COLS == 128 || COLS == 256, "tile rows of 128, 256 or 512 bytes");
     static __device__ __forceinline__ int swizzle(int r) { return swz<(COLS > 128 ? 128 : COLS)>(r); }
 };
 
