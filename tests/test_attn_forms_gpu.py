@@ -33,6 +33,31 @@ def test_forms(gpu, case, dtype):
     assert not bad, bad
 
 
+# B, S, Hq, Hkv, causal; the kernels that the rules for 256 compute units give D 128 there: short grids on the
+# split HIP forms, full ones and the smallest calls on the assembly, each stage by its own grid
+PATHS = [((1, 770, 3, 1, True), "fwd_hip", "dq_hip", "dkdv_hip"), ((2, 800, 8, 4, True), "fwd_hip", "dq_hip", "dkdv_hip"),
+         ((4, 257, 16, 16, False), "fwd_hip", "dq_hip", "dkdv_asm"), ((3, 600, 33, 3, True), "fwd_asm", "dq_asm", "dkdv_hip"),
+         ((4, 512, 4, 2, True), "fwd_asm", "dq_hip", "dkdv_hip"), ((4, 1024, 16, 16, True), "fwd_asm", "dq_asm", "dkdv_asm")]
+
+
+@pytest.mark.parametrize("dtype", ("f16", "bf16"))
+@pytest.mark.parametrize("shape,fwd,dq,dkdv", PATHS, ids=["B%d-S%d-%d-%d-c%d" % p[0] for p in PATHS])
+def test_d128_kernels_of_the_rule(gpu, shape, fwd, dq, dkdv, dtype):
+    import torch
+    from tokamak_amd import attn
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the shapes are at the rules' lines for 256 compute units")
+    B, S, Hq, Hkv, causal = shape
+    log(f"[case] kernels of B{B} S{S} Hq{Hq} Hkv{Hkv} D128 {dtype}")
+    dt = torch.float16 if dtype == "f16" else torch.bfloat16
+    qkv = torch.randn((B, S, (Hq + 2 * Hkv) * 128), device=gpu).to(dt)
+    o, lse = attn.gqa_fwd(qkv, B, S, Hq, Hkv, 128, causal=causal)
+    assert attn.last_kernels() == [fwd]
+    attn.gqa_bwd(qkv, o, torch.randn_like(o), lse, B, S, Hq, Hkv, 128, causal=causal)
+    assert attn.last_kernels() == [dq, dkdv]
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("S,where", ((300, 280), (300, 5), (1100, 700)))
 def test_nan_key_reaches_output_from_every_group(gpu, S, where):
     """A NaN in one key's V makes every row that sees the key NaN, whichever group of waves walks its

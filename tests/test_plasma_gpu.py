@@ -186,8 +186,9 @@ def test_plasma_config4_swiglu(gpu):
 @pytest.mark.parametrize("rows", (1, 33, 1027, 4099))
 @pytest.mark.parametrize("c", (dict(C=64, chain=["RMSNorm", "LayerScale"], acc=6),
                                dict(C=256, chain=["Bias", "Add", "RMSNorm"], acc=7),
-                               dict(C=1376, twin=True, left=["SiLU"], right=[], chain=[], acc=1)),
-                         ids=lambda c: f"C{c['C']}")
+                               dict(C=1376, twin=True, left=["SiLU"], right=[], chain=[], acc=1),
+                               dict(C=1376, chain=["Bias", "LayerScale"], acc=6)),   # 4099 rows: bands of 8, two passes
+                         ids=lambda c: f"C{c['C']}" + ("" if c["chain"] != ["Bias", "LayerScale"] else "-partials"))
 def test_plasma_row_bands(gpu, c, rows):
     """Rows less and more than a pass of one block, and bands of several passes (narrow rows take 32 and
     8 rows a pass, wide ones 4), with and without parameter partials."""
